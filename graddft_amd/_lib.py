@@ -13,6 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libgdx.so")
 
 GDX_FP64, GDX_FP32, GDX_BF16X6 = 0, 1, 2
+GDX_AO_LOW = 16
 GDX_FUNC_B3LYP, GDX_FUNC_NEURAL_B3LYP, GDX_FUNC_B3LYP_NEURAL_CORR, GDX_FUNC_LINEAR = 0, 1, 2, 3
 GDX_CORR_VWN5, GDX_CORR_PW92 = 0, 1
 GDX_STATUS_EIGH_NOT_CONVERGED, GDX_STATUS_NONFINITE_ENERGY, GDX_STATUS_CHARGE = 1, 2, 4

@@ -18,8 +18,14 @@
 // FP32 planes: X is formed in FP64 (AO values widened, D as it is), because rho is a sum that cancels;
 // U and the derivatives are split into three bf16 terms (gdx_gemm_split.h).  With X on split products,
 // too, the kernel is a third faster, but an MFMA aligns its 32 products to the largest and cuts what is
-// below, which biases rho (E_xc of an alkane by -1e-8, FP32 MFMA +-1e-8, this way 3e-10 .. 3e-9; dE/dD
-// of n = 560 by 1e-7 .. 9e-7, FP32 MFMA 5e-8 .. 4e-7, this way 2e-8 .. 3e-8).
+// below, which biases rho and moves dE/dD of n = 560 by 1e-7 .. 9e-7 (FP32 MFMA 5e-8 .. 4e-7, this way
+// 2e-8 .. 3e-8).
+// LOW: the FP32 planes come with d = phi - float(phi) in bf16, and rho = X . (float(phi) + 2 d), which
+// is phi D phi to first order in d for a symmetric D.  All points of a shell around a nucleus have
+// nearly the same core functions, so their rounding does not average out over the grid: without d, E_xc
+// of water, alkanes and benzene (6-31G*, def2-SVP, levels 1 and 2, B3LYP and neural) moves by
+// -1.7e-8 .. +1.4e-8 of itself, alike for all molecules of a basis and level.  With it 1e-9 remains, from
+// phi in the gradients; the derivatives and the Laplacian, rounded too, move it by under 5e-10.
 //
 // Bound by the MFMA rate at FP64 (n = 190, 144k points, one spin: 1.02 -> 0.67 ms, 53% of it; the rest
 // waits for loads with two waves a SIMD) and by load latency at FP32, where every chunk reads the planes
@@ -32,7 +38,7 @@
 namespace gdx {
 
 struct DensMol {
-  const void* ao;      // (5, npts_pad, nP) planes in the element type
+  const void* ao;      // (5, npts_pad, nP) planes in the element type; LOW: then a bf16 plane phi - float(phi)
   void* pack;          // D and U fragments of the spins, dens_pack_bytes each
   long row0, dm_off;   // first row in the per-point arrays, first element in the density matrices
   int npts_pad, nP, n;
@@ -185,7 +191,7 @@ struct DensDouble {
   }
 };
 // Grid: dens_blocks; dens_part rows are DENS_STRIDE doubles, out_rows a spin.
-template <typename T>
+template <typename T, bool LOW>
 __global__ __launch_bounds__(256, 2) void density_kernel(const DensMol* __restrict__ mols, int nmol, const DensMol one,
                                                          int nspin, size_t out_rows, double* __restrict__ dens_part) {
   typedef typename MfmaT<T>::acc_t acc_t;
@@ -202,6 +208,8 @@ __global__ __launch_bounds__(256, 2) void density_kernel(const DensMol* __restri
   const int nch = dens_chunks(nP), nks = dens_ksteps<T>(nP);
   const size_t plane = (size_t)M.npts_pad * nP;
   const gptr<T> rows = (gptr<T>)M.ao + (size_t)(tile * DN_PT + wave * 16) * nP;   // this wave's 16 points
+  static_assert(!LOW || sizeof(T) == 4, "the remainder of phi goes with FP32 planes");
+  const gptr<char> lows = (gptr<char>)((gptr<T>)M.ao + 5 * plane) + (size_t)(tile * DN_PT + wave * 16) * nP * 2;
   const gptr<char> pack = (gptr<char>)M.pack + s * dens_pack_bytes<T>(nP);
 
   f4 ra[4][NV], rb[NB];
@@ -343,11 +351,14 @@ __global__ __launch_bounds__(256, 2) void density_kernel(const DensMol* __restri
     // contraction with the AO values at the chunk's columns, four a lane, one 16-byte vector of each
     // plane at a time and one ahead
     constexpr int VE = 16 / sizeof(T);   // columns a vector
+    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
     f4 rc[5];
+    bf4 rl = (bf4)(__bf16)0.f;
     auto cload = [&](int v) {
-      const unsigned at = (r * nP + (m * DN_CB + v / CV) * 16 + 4 * g + v % CV * VE) * (unsigned)sizeof(T);
+      const unsigned at = r * nP + (m * DN_CB + v / CV) * 16 + 4 * g + v % CV * VE;
 #pragma unroll
-      for (int k = 0; k < 5; ++k) rc[k] = row_load<f4>(rows + k * plane, at);
+      for (int k = 0; k < 5; ++k) rc[k] = row_load<f4>(rows + k * plane, at * (unsigned)sizeof(T));
+      if (LOW) rl = row_load<bf4>(lows, at * 2);
     };
     cload(0);
 #pragma unroll
@@ -358,12 +369,13 @@ __global__ __launch_bounds__(256, 2) void density_kernel(const DensMol* __restri
       vec_t x[5];
 #pragma unroll
       for (int k = 0; k < 5; ++k) x[k] = __builtin_bit_cast(vec_t, rc[k]);
+      const bf4 xl = rl;
       if (v + 1 < jn * CV) cload(v + 1);
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
         const int q = v % CV * VE + e;
         const double x0 = acc0[j][q], gx = x[1][e], gy = x[2][e], gz = x[3][e];
-        part[0] += x0 * (double)x[0][e];
+        part[0] += x0 * (LOW ? (double)x[0][e] + 2.0 * (double)(float)xl[e] : (double)x[0][e]);
         part[1] += x0 * gx;
         part[2] += x0 * gy;
         part[3] += x0 * gz;

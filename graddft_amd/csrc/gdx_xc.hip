@@ -775,8 +775,9 @@ int validate(const gdx_xc_desc* d) {
               "unknown functional kind");
   GDX_REQUIRE(d->correlation == GDX_CORR_VWN5 || d->correlation == GDX_CORR_PW92,
               "correlation must be GDX_CORR_VWN5 or GDX_CORR_PW92");
-  if (d->precision != GDX_FP64 && d->precision != GDX_FP32 && d->precision != GDX_BF16X6) {
-    set_error("unknown precision (GDX_FP64, GDX_FP32, GDX_BF16X6)");
+  const int prec = d->precision & ~GDX_AO_LOW;
+  if ((prec != GDX_FP64 && prec != GDX_FP32 && prec != GDX_BF16X6) || d->precision == (GDX_FP64 | GDX_AO_LOW)) {
+    set_error("unknown precision (GDX_FP64, GDX_FP32, GDX_BF16X6; GDX_AO_LOW with the latter two)");
     return GDX_ERR_UNSUPPORTED;
   }
   if (is_neural(*d)) {
@@ -797,7 +798,7 @@ inline unsigned nblocks64(long n) { return (unsigned)((n + 63) / 64); }
 template <typename T> const char* tname(const char* f64, const char* f32) { return sizeof(T) == 8 ? f64 : f32; }
 template <typename T>
 const char* gname(const gdx_xc_desc& d, const char* f64, const char* f32, const char* bf16x6) {
-  return sizeof(T) == 8 ? f64 : (d.precision == GDX_BF16X6 ? bf16x6 : f32);
+  return sizeof(T) == 8 ? f64 : ((d.precision & ~GDX_AO_LOW) == GDX_BF16X6 ? bf16x6 : f32);
 }
 
 // The hidden-layer products, C = epi(A W) (or A W^T for TB) over M rows and the split-K weight
@@ -977,8 +978,16 @@ void launch_density(const Ctx& c, const T* ao, const double* mats, bool tangent,
     pblocks = (int)((dens_pack_threads<T>(d.nao_pad, nspin) + 255) / 256);
   }
   GDX_LAUNCH("pad_dm", dens_pack_kernel<T>, dim3(pblocks), dim3(256), 0, st, mols, nmol, one, nspin, mats);
-  GDX_LAUNCH(tname<T>("density_f64", "density_f32"), density_kernel<T>, dim3(blocks), dim3(NT), 0, st, mols, nmol, one,
-             nspin, (size_t)d.npts_pad, out);
+  const char* nm = tname<T>("density_f64", "density_f32");
+  if constexpr (sizeof(T) == 4) {
+    if (d.precision & GDX_AO_LOW) {
+      GDX_LAUNCH(nm, (density_kernel<T, true>), dim3(blocks), dim3(NT), 0, st, mols, nmol, one, nspin,
+                 (size_t)d.npts_pad, out);
+      return;
+    }
+  }
+  GDX_LAUNCH(nm, (density_kernel<T, false>), dim3(blocks), dim3(NT), 0, st, mols, nmol, one, nspin, (size_t)d.npts_pad,
+             out);
 }
 
 // V_xc products of one molecule (`one`, mols null) or a batch, reduced into d_rdm1

@@ -34,7 +34,9 @@ import torch
 from . import _lib
 from .molecule import Molecule
 
-PRECISIONS = {"fp64": _lib.GDX_FP64, "fp32": _lib.GDX_FP32, "bf16x6": _lib.GDX_BF16X6}
+# the library's precision of a plan over ao_planes_for's planes
+PRECISIONS = {"fp64": _lib.GDX_FP64, "fp32": _lib.GDX_FP32 | _lib.GDX_AO_LOW,
+              "bf16x6": _lib.GDX_BF16X6 | _lib.GDX_AO_LOW}
 
 
 @dataclass(frozen=True)
@@ -63,13 +65,19 @@ AUTOTUNE = True
 
 def ao_planes_for(m: Molecule, precision: str) -> torch.Tensor:
     """AO planes in the element type of a precision: the FP64 planes, or their FP32 copy
-    (made once and cached on the molecule)."""
+    (made once and cached on the molecule), whose storage goes on with the bf16 plane of what
+    rounding phi to FP32 left (GDX_AO_LOW)."""
     if precision == "fp64":
         return m.ao_planes
     key = ("ao_planes_f32", m.ao_planes.data_ptr())
     a = m.cache.get(key)
     if a is None:
-        a = m.ao_planes.to(torch.float32)
+        p = m.ao_planes
+        n = p[0].numel()   # even: the padded rows are a multiple of 64
+        buf = torch.empty(5 * n + n // 2, dtype=torch.float32, device=p.device)
+        a = buf[:5 * n].view(p.shape)
+        a.copy_(p)
+        torch.sub(p[0], a[0], out=buf[5 * n:].view(torch.bfloat16).view(p.shape[1:]))
         m.cache[key] = a
     return a
 

@@ -35,6 +35,11 @@ enum {
  *             six products on v_mfma_f32_16x16x32_bf16, FP32 sums (at least FP32's accuracy)
  *  GDX_BF16X6 the same kernels as GDX_FP32. */
 enum { GDX_FP64 = 0, GDX_FP32 = 1, GDX_BF16X6 = 2 };
+/* Or-ed into GDX_FP32 or GDX_BF16X6: the buffer of the five float AO planes goes on with a plane
+ * (npts_pad, nao_pad) of bf16 values phi - (float)phi, with which rho is formed.  Without it the
+ * rounding of phi moves E_xc by up to 2e-8 of itself: the core functions are nearly constant on every
+ * shell of grid points around a nucleus, so that it does not average out. */
+enum { GDX_AO_LOW = 16 };
 
 /* Functional kinds evaluated on the grid.
  *  GDX_FUNC_B3LYP        E = sum_r w * (0.8 e_lda + 0.72 e_b88 + 0.19 e_vwn + 0.81 e_lyp)
@@ -94,7 +99,7 @@ int gdx_xc_workspace_size(const gdx_xc_desc* desc, size_t* bytes);
  * as in compute_densities / compute_coefficient_inputs (:160-217) and
  * grad_dft/molecule.py:388-502.
  * ao: gdx_ao_eval output in the element type of desc->precision (double planes for
- * GDX_FP64, float planes otherwise); weights (npts_pad) grid weights, zero past npts;
+ * GDX_FP64, float planes otherwise, with GDX_AO_LOW the bf16 plane after them); weights (npts_pad) grid weights, zero past npts;
  * rdm1 (2, nao, nao); params: flat MLP parameters [W0 (nc,h), b0 (h), W1 (h,h), b1, ...,
  * W_last (h,nd), b_last] (NULL for GDX_FUNC_B3LYP).  exc: one device double.
  * The workspace keeps what gdx_xc_backward needs; do not touch it in between. */

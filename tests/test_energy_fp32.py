@@ -1,0 +1,53 @@
+"""FP32 energies against the FP64 path on the same, unrounded inputs.  The grid's points lie on shells
+around the nuclei on which the core functions are nearly constant, so what is rounded once for all
+points of a shell -- phi -- does not average out: FP32 planes carry the remainder of phi."""
+import numpy as np
+import pytest
+import torch
+
+
+def _alkane(atoms, basis, level, seed=3, align=256):
+    from graddft_amd.interface import geometry
+    from graddft_amd.interface.builder import molecule_from_geometry
+    sym, xyz = geometry.alkane(np.random.default_rng(seed), atoms)
+    return molecule_from_geometry(sym, xyz, basis, level, npts_align=align)
+
+
+def test_fp32_planes_carry_the_remainder_of_phi():
+    from types import SimpleNamespace
+    from graddft_amd.functional import ao_planes_for
+    planes = torch.randn(5, 64, 16, dtype=torch.float64)
+    m = SimpleNamespace(ao_planes=planes, cache={})
+    a = ao_planes_for(m, "fp32")
+    assert a.dtype == torch.float32 and torch.equal(a, planes.float())
+    low = torch.empty(0, dtype=torch.float32).set_(a.untyped_storage())[5 * 64 * 16:].view(torch.bfloat16)
+    phi = a[0].double() + low.double().view(64, 16)
+    # FP32 rounds by 2^-24 at most, bf16 keeps eight bits of that
+    assert float(((phi - planes[0]).abs() / planes[0].abs()).max()) <= 2.0 ** -32
+    assert ao_planes_for(m, "bf16x6") is a and ao_planes_for(m, "fp64") is planes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("basis,level", [("def2-svp", 1), ("def2-svp", 2), ("6-31g*", 1), ("6-31g*", 2)])
+def test_rho_and_grid_energies(basis, level):
+    from graddft_amd import B3LYP_GRID
+    from graddft_amd.batch import XCBatchPlan
+    mols = [_alkane(c, basis, level) for c in (1, 2, 4)]
+    E = {}
+    for p in ("fp64", "fp32", "bf16x6"):
+        plan = XCBatchPlan(B3LYP_GRID, mols, p)
+        e = torch.empty(len(mols), dtype=torch.float64, device="cuda")
+        plan.forward(plan.concat([m.rdm1 for m in mols]), None, e)
+        E[p] = e.cpu()
+        plan.close()
+    for p in ("fp32", "bf16x6"):
+        print(f"case: {basis} level {level} {p}:", ((E[p] - E["fp64"]) / E["fp64"]).tolist(), flush=True)
+        # phi in the gradients and the rounded derivatives move E_xc by 1.5e-9 of itself at most, the
+        # products of the kinetic term by less than that
+        assert float(((E[p] - E["fp64"]) / E["fp64"]).abs().max()) <= 3e-9
+    m = mols[1]
+    for restricted in (True, False):
+        mm = m.replace(restricted=restricted)
+        rho = {p: B3LYP_GRID.plan(mm, p).densities(mm.rdm1)[:, :, 0] for p in ("fp64", "fp32")}
+        # the remainder's 2^-9 of 2^-24 twice; what rounding phi alone leaves is 3e-8
+        assert float((rho["fp32"] - rho["fp64"]).norm() / rho["fp64"].norm()) <= 2.0 ** -31
