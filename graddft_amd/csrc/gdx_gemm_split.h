@@ -6,9 +6,12 @@
 // and a product a.b is formed from the six terms whose order is >= 2^-18 of it:
 //   a_h b_h + a_h b_m + a_m b_h + a_h b_l + a_m b_m + a_l b_h,
 // accumulated in FP32.  The dropped terms (2^-27) are below FP32's own rounding (2^-24), and an
-// MFMA adds 32 products at a time where the FP32 instruction adds four, so the sums round less:
-// dE/dtheta of the 3 x 256 network on benzene is 6e-8 from FP64 (FP32 MFMA 2.5e-7), dE/dD
-// 4.2e-8 (3.9e-8: the rounding of D).  A two-term split with three products is not enough (E_xc moves by 5e-6 Ha).
+// MFMA adds 32 products at a time where the FP32 instruction adds four, so the sums round less often,
+// though not to nearest (mfma_split): dE/dtheta of the 3 x 256 network on benzene is 6e-8 from FP64 (FP32
+// MFMA 2.5e-7), dE/dD 4.2e-8 (3.9e-8: the rounding of D); total energies of 32 batches of alkanes, all
+// widths, are 4e-10 (rms, at most 1e-9) from FP64, half of them up and half down, where FP32 MFMA in the
+// layers and the densities left 8e-9.  A two-term split with three products is not enough (E_xc moves by
+// 5e-6 Ha).
 //
 // The weights are split from their FP64 masters once per evaluation (pack_weights_kernel), in the
 // order a wave reads them as MFMA operands, and stay in L2; activations are split once per block
@@ -44,21 +47,31 @@ __device__ __forceinline__ void split8(const float* x, bf8& h, bf8& m, bf8& l) {
 }
 
 // acc[i] += the six products of 16 x 16 x 32 steps a . b[i] for NI blocks.  A block's products are
-// summed from zero, smallest first, and added to the running sum once: every MFMA rounds its whole
-// accumulator, so a chain of all six through acc would round it six times a step, as often as FP32
-// MFMAs do.  The blocks' chains are interleaved (an MFMA waits for the previous one of its chain).
-template <int NI>
+// summed from zero and added to the running sum once: every MFMA rounds its whole accumulator, so a
+// chain of all six through acc would round it six times a step, as often as FP32 MFMAs do.  The blocks'
+// chains are interleaved (an MFMA waits for the previous one of its chain).
+// LEAD: the leading product has a sum of its own.  An MFMA aligns its addends to the largest and cuts
+// towards minus infinity what is below: for normally distributed factors -0.19 x 2^-24 of the largest
+// product on average where the leading product joins the chain of the small ones, 0.004 where it does
+// not.  In the layers of the energy that is a shift of every unit alike at all points, which moves E_xc
+// by 5e-9 of itself; gradients, rounded to 4e-8 anyway, are spared its registers (3% of a benzene
+// 6-31G* step).
+template <int NI, bool LEAD>
 __device__ __forceinline__ void mfma_split(const bf8 (&a)[3], const bf8 (&b)[NI][3], f4 (&acc)[NI]) {
   constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
-  f4 t[NI];
+  f4 t[NI], lead[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) t[i] = (f4)0.f;
 #pragma unroll
-  for (int p = 0; p < 6; ++p)
+  for (int p = 0; p < (LEAD ? 5 : 6); ++p)
 #pragma unroll
     for (int i = 0; i < NI; ++i) t[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[PA[p]], b[i][PB[p]], t[i], 0, 0, 0);
+  if (LEAD) {
 #pragma unroll
-  for (int i = 0; i < NI; ++i) acc[i] += t[i];
+    for (int i = 0; i < NI; ++i) lead[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[i][0], (f4)0.f, 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) acc[i] += LEAD ? lead[i] + t[i] : t[i];
 }
 
 // the same chain of one block through c (which FP64 accumulators then take)
@@ -184,7 +197,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(int M, int h, const 
         for (int p = 0; p < 3; ++p) hb[i][p] = *(const bf8*)&As[cur][p][(g * GS_ROWS + i * 16 + (r ^ (2 * g))) * 8];
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
-        mfma_split<4>(w[j], hb, acc[j]);
+        mfma_split<4, EPI == EPI_BIAS_ELU>(w[j], hb, acc[j]);
         wload(nxt, j, w[j]);   // the next step's fragments, into the registers just read
       }
       cur ^= 1;
@@ -312,7 +325,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_split_kernel(int h, const float*
 #pragma unroll
         for (int p = 0; p < 3; ++p) gb[p] = *(const bf8*)&Bs[p][g][(wf + j * 16 + r) * 8];
         // MFMA rows: features f; columns: inputs i (blocks past h only multiply zeros)
-        if (niv > 0) mfma_split<4>(gb, ha, acc[j]);
+        if (niv > 0) mfma_split<4, false>(gb, ha, acc[j]);
       }
     }
     __syncthreads();
