@@ -17,6 +17,7 @@
 #pragma once
 #include "gdx_common.h"
 #include "gdx_gemm.h"
+#include "gdx_skinny.h"
 
 namespace gdx {
 
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(256) void delta_wgrad_rows_kernel(const T* __restri
 template <typename T, bool HEAD>
 __global__ __launch_bounds__(256) void rowdot_mfma_kernel(int rows, int K, const T* __restrict__ A,
                                                           const T* __restrict__ Bt, T* __restrict__ out, int nout,
-                                                          const T* __restrict__ bias, const double* __restrict__ E,
+                                                          const double* __restrict__ bias, const double* __restrict__ E,
                                                           const double* __restrict__ weights, int npts,
                                                           double* __restrict__ eps_part, int head_mode) {
   static_assert(RD_ROWS == 64, "one 16-row group per wave of a 256-thread block");
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(256) void rowdot_mfma_kernel(int rows, int K, const
         const int rr = r0 + hr;
         double prod = 0.0;
         if (rr < npts && ho < nout) {
-          const double zz = zs[wave][hr][ho] + (double)bias[ho];
+          const double zz = head_z<T>(zs[wave][hr], ho, nout) + bias[ho];
           const double c = head_coef(zz, head_mode, ho);
           out[(size_t)rr * nout + ho] = (T)c;
           prod = c * E[(size_t)rr * nout + ho];
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(256) void rowdot_mfma_kernel(int rows, int K, const
         if (rr < npts) {
           double eps = 0.0;
           for (int o = 0; o < nout; ++o) {
-            const double zz = zs[wave][lane][o] + (double)bias[o];
+            const double zz = head_z<T>(zs[wave][lane], o, nout) + bias[o];
             const double c = head_coef(zz, head_mode, o);
             out[(size_t)rr * nout + o] = (T)c;
             eps += c * E[(size_t)rr * nout + o];

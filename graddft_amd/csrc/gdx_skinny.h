@@ -18,12 +18,21 @@ namespace gdx {
 
 constexpr int SK_KC = 64;  // K chunk staged per LDS pass
 
+// output o of a row's 16 products: in FP32 the weights' remainders follow in column nd + o (an infinite
+// activation times a zero remainder is left out)
+template <typename T>
+__device__ __forceinline__ double head_z(const double* z, int o, int nd) {
+  if (sizeof(T) == 8) return z[o];
+  const double lo = z[nd + o];
+  return isfinite(lo) ? z[o] + lo : z[o];
+}
+
 template <typename T, bool HEAD>
 __global__ __launch_bounds__(256) void skinny_out16_kernel(
     int M, int K, const T* __restrict__ A, int lda, const T* __restrict__ Bt,
     T* __restrict__ C16, int ldc, int ncols,
     // head epilogue
-    const T* __restrict__ bias, int nd, const double* __restrict__ E,
+    const double* __restrict__ bias, int nd, const double* __restrict__ E,
     const double* __restrict__ weights, int npts, double* __restrict__ eps_part, int head_mode = 0) {
   typedef typename MfmaT<T>::acc_t acc_t;
   __shared__ T As[64][SK_KC + 2];
@@ -80,7 +89,7 @@ __global__ __launch_bounds__(256) void skinny_out16_kernel(
     if (r < npts) {
       double eps = 0.0;
       for (int o = 0; o < nd; ++o) {
-        const double z = zs[tid][o] + (double)bias[o];
+        const double z = head_z<T>(zs[tid], o, nd) + bias[o];
         const double c = head_coef(z, head_mode, o);
         C16[(size_t)r * ldc + o] = (T)c;
         eps += c * E[(size_t)r * nd + o];

@@ -199,13 +199,15 @@ __global__ __launch_bounds__(NT) void point_fwd_kernel(
 }
 
 // Row-wise products against at most 16 weight rows, for the MLP's narrow edges:
-//   v[r][f] = sum_{j < kj} A[r][j] Wt[j][f]   (A with row stride 16, Wt (16 x h) in LDS)
+//   v[r][f] = sum_{j < kj} A[r][j] Wt[j][f]   (A with row stride 16, Wt (16 x h) in LDS);
+// ER_LAYER0 in FP32 adds the weights' remainders in rows EDGE_LO0 + j
 //   ER_LAYER0:    out = ELU(v + b[f])             (first layer, forward)
 //   ER_TANGENT0:  out = v * elu'(Y[r][f])         (first layer, tangent)
 //   ER_DELTA:     out = v * elu'(Y[r][f])         (last layer's input adjoint)
 //   ER_RAW:       out = v
 // elu'(z) is taken from Y = ELU(z).  Each thread forms 8 consecutive features of one row
 // (16- / 32-byte stores); a block covers ER_ROWS rows.
+constexpr int EDGE_LO0 = 8;
 enum { ER_LAYER0 = 0, ER_TANGENT0 = 1, ER_DELTA = 2, ER_RAW = 3 };
 constexpr int ER_ROWS = 64;
 
@@ -251,6 +253,11 @@ __global__ __launch_bounds__(NT) void edge_rows_kernel(const T* __restrict__ A, 
     v8 v;
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (T)0;
+    if (MODE == ER_LAYER0 && sizeof(T) == 4) {
+#pragma unroll
+      for (int j = 0; j < EDGE_LO0; ++j)
+        if (j < kj) v += a[j] * *(const v8*)&Ws[EDGE_LO0 + j][f0];
+    }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       if (j < kj) {
@@ -275,7 +282,10 @@ __global__ __launch_bounds__(NT) void edge_rows_kernel(const T* __restrict__ A, 
 // ----------------------------------------------------------------- MLP head ----
 
 // Padded weight tiles for the skinny kernels: WT16 (16 x h) rows o < nd = W_last[:, o];
-// W016 (16 x h) rows j < nc = W0[j, :]; every other row zero.
+// W016 (16 x h) rows j < nc = W0[j, :]; every other row zero, but in FP32 rows nd + o and EDGE_LO0 + j
+// hold what rounding those weights left, which the first layer and the head of the energy add (the rows
+// are in the 16-wide tiles anyway).  A weight's rounding is the same at every point: without the
+// remainders E_xc of alkanes and benzene moves by up to 1e-8 of itself.
 template <typename T>
 __global__ void prep_edge_weights_kernel(const double* __restrict__ W0, int nc,
                                          const double* __restrict__ Wl, int nd, int h,
@@ -283,8 +293,14 @@ __global__ void prep_edge_weights_kernel(const double* __restrict__ W0, int nc,
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= 16 * h) return;
   const int row = i / h, f = i % h;
-  W016[i] = (T)(row < nc ? W0[row * h + f] : 0.0);
-  WT16[i] = (T)(row < nd ? Wl[f * nd + row] : 0.0);
+  constexpr bool LO = sizeof(T) == 4;
+  auto part = [&](double w, bool lo) {
+    const T hi = (T)w;
+    return !lo ? hi : isfinite(hi) ? (T)(w - (double)hi) : (T)0;
+  };
+  const int j = LO && row >= EDGE_LO0 ? row - EDGE_LO0 : row, o = LO && row >= nd ? row - nd : row;
+  W016[i] = j < nc ? part(W0[j * h + f], j != row) : (T)0;
+  WT16[i] = o < nd ? part(Wl[f * nd + o], o != row) : (T)0;
 }
 
 // Adjoint seeds, one thread per point.  g = g_exc clip(w) [|eps| > 1e-30];
@@ -1171,11 +1187,11 @@ int forward_impl(const Ctx& c, const T* ao, const double* weights, const double*
     if (rows_path(h)) {
       nred = (Np + RD_ROWS - 1) / RD_ROWS;
       GDX_LAUNCH("head_fwd", (rowdot_mfma_kernel<T, true>), dim3(nred), dim3(NT), 0, st, Np, h,
-                 H + (size_t)(nl - 1) * L.hstride, WT16, c.P<T>(L.C), d.mlp_nd, plp + po.b[nl], c.P<double>(L.E),
+                 H + (size_t)(nl - 1) * L.hstride, WT16, c.P<T>(L.C), d.mlp_nd, params + po.b[nl], c.P<double>(L.E),
                  weights, d.npts, c.P<double>(L.eps_part), hmode);
     } else {
       GDX_LAUNCH("head_fwd", (skinny_out16_kernel<T, true>), dim3(Np / 64), dim3(NT), 0, st, Np, h,
-                 H + (size_t)(nl - 1) * L.hstride, h, WT16, c.P<T>(L.C), d.mlp_nd, d.mlp_nd, plp + po.b[nl],
+                 H + (size_t)(nl - 1) * L.hstride, h, WT16, c.P<T>(L.C), d.mlp_nd, d.mlp_nd, params + po.b[nl],
                  d.mlp_nd, c.P<double>(L.E), weights, d.npts, c.P<double>(L.eps_part), hmode);
       nred = Np / 64;
     }

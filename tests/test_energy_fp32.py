@@ -51,3 +51,29 @@ def test_rho_and_grid_energies(basis, level):
         rho = {p: B3LYP_GRID.plan(mm, p).densities(mm.rdm1)[:, :, 0] for p in ("fp64", "fp32")}
         # the remainder's 2^-9 of 2^-24 twice; what rounding phi alone leaves is 3e-8
         assert float((rho["fp32"] - rho["fp64"]).norm() / rho["fp64"].norm()) <= 2.0 ** -31
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("basis,level,h,layers,seed", [("def2-svp", 1, 16, 2, 1), ("def2-svp", 2, 16, 4, 2),
+                                                       ("6-31g*", 1, 96, 3, 2), ("6-31g*", 2, 128, 3, 5),
+                                                       ("def2-svp", 1, 192, 2, 7), ("6-31g*", 1, 256, 4, 8)])
+def test_batch_energies_of_a_network(basis, level, h, layers, seed):
+    """Total energies of a ragged batch: beside phi, the first and the last layer's weights are rounded
+    alike at every point, and come with their remainders."""
+    from graddft_amd import MLPSpec, NeuralFunctional, batch_energy_predictor
+    from graddft_amd.interface import geometry
+    from graddft_amd.interface.builder import molecule_from_geometry
+    rng = np.random.default_rng(seed)
+    mols = []
+    for c in (1, 2, 3):
+        sym, xyz = geometry.alkane(rng, c)
+        mols.append(molecule_from_geometry(sym, xyz, basis, level, with_eri=True, npts_align=256))
+    f = NeuralFunctional(MLPSpec(nc=6, h=h, n_hidden=layers, nd=4))
+    theta = f.init(seed=seed)
+    e = {p: torch.stack(list(batch_energy_predictor(f, precision=p)(theta, mols)[0])).double().cpu()
+         for p in ("fp64", "fp32")}
+    off = (e["fp32"] - e["fp64"]) / e["fp64"]
+    print(f"case: {basis} level {level} {layers} x {h}:", off.tolist(), flush=True)
+    # E_xc, a quarter of the energy or less, is left 3e-9 by the planes (above) and as much by the
+    # roundings within the network; they have no common sign
+    assert float(off.abs().max()) <= 1e-9
