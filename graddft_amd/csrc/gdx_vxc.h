@@ -29,14 +29,15 @@ namespace gdx {
 
 struct VxcMol {
   const void* ao;      // (5, npts_pad, nP) planes in the element type
-  float* z;            // FP32: (nsv, npts_pad, nP) Z
-  float* u;            // FP32: (nsv, npts_pad) u as a pair (high, low)
+  float* z;            // FP32: (nsv, slab, nP) Z of the current slab
+  float* u;            // FP32: (nsv, slab) u as a pair (high, low)
   double* part;        // partial sums, (slots, nsv, nP, nP): see vxc_reduce_kernel
   long row0;           // first row of this molecule in every spin plane of the potentials
   long out_off;        // first element of its (2, n, n) output
   int npts_pad, nP, n;
+  int slab;            // points a launch (FP32; a multiple of 64), all of them in FP64
   int tb, nf, rem;     // 16-wide blocks a tile, full tiles an edge, blocks of the last, ragged one
-  int ch[4], nch[4];   // points per chunk and chunks of the item classes
+  int ch[4], nch[4];   // points per chunk and chunks a slab of the item classes
   int blk0, zblk0, rblk0;   // first block in the product, Z and reduction launches
 };
 
@@ -100,29 +101,30 @@ __device__ __forceinline__ VxcMol vxc_find(const VxcMol* __restrict__ mols, int 
   return u.m;
 }
 
-// FP32: Z of every point, column and spin, once instead of once per tile row, and u as FP32 pairs; four
-// columns of a row a thread.  HBM-bound: reads the five planes once, writes nsv.
+// FP32: Z of every point of a slab, column and spin, once instead of once per tile row, and u as FP32
+// pairs; four columns of a row a thread.  HBM-bound: reads the five planes once, writes nsv.
 __global__ __launch_bounds__(256) inline void vxc_zform_kernel(const VxcMol* __restrict__ mols, int nmol,
                                                                const VxcMol one, const double* __restrict__ vpt,
-                                                               size_t vpt_rows, int nsv) {
+                                                               size_t vpt_rows, int nsv, int slab) {
   const VxcMol M = vxc_find<&VxcMol::zblk0>(mols, nmol, one, blockIdx.x);
-  const long i = ((long)(blockIdx.x - M.zblk0) * 256 + threadIdx.x) * 4;   // npts_pad nP is a multiple of 1024
-  const long plane = (long)M.npts_pad * M.nP;
-  const gptr<float> ao = (gptr<float>)M.ao + i;
+  const long i = ((long)(blockIdx.x - M.zblk0) * 256 + threadIdx.x) * 4;   // slab nP is a multiple of 1024
+  const long plane = (long)M.npts_pad * M.nP, zplane = (long)M.slab * M.nP;
+  const long r0 = (long)slab * M.slab, r = i / M.nP;
+  if (r0 + r >= M.npts_pad) return;   // the last slab may be shorter
+  const gptr<float> ao = (gptr<float>)M.ao + r0 * M.nP + i;
   const f4 p = *(gptr<f4>)ao, x = *(gptr<f4>)(ao + plane), y = *(gptr<f4>)(ao + 2 * plane),
            z = *(gptr<f4>)(ao + 3 * plane), l = *(gptr<f4>)(ao + 4 * plane);
-  const long r = i / M.nP;
   for (int s = 0; s < nsv; ++s) {
-    const double* v = vpt + ((size_t)s * vpt_rows + M.row0 + r) * VPT_STRIDE;
+    const double* v = vpt + ((size_t)s * vpt_rows + M.row0 + r0 + r) * VPT_STRIDE;
     const double v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3], v4 = v[4];
     f4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (float)(v0 * (double)p[e] + v1 * (double)x[e] + v2 * (double)y[e] +
                                               v3 * (double)z[e] + v4 * (double)l[e]);
-    *(gptr_w<f4>)((gptr_w<float>)M.z + (long)s * plane + i) = o;
+    *(gptr_w<f4>)((gptr_w<float>)M.z + s * zplane + i) = o;
     if (i % M.nP == 0) {
       const float h = (float)v[5];
-      gptr_w<float> w = (gptr_w<float>)M.u + 2 * ((long)s * M.npts_pad + r);
+      gptr_w<float> w = (gptr_w<float>)M.u + 2 * ((long)s * M.slab + r);
       w[0] = h;
       w[1] = (float)(v[5] - (double)h);
     }
@@ -136,7 +138,7 @@ struct VxcItem {
 };
 
 template <typename T>
-__device__ __forceinline__ bool vxc_item(const VxcMol& M, int nsv, VxcItem& it) {
+__device__ __forceinline__ bool vxc_item(const VxcMol& M, int nsv, int slab, VxcItem& it) {
   const int local = blockIdx.x - M.blk0, xcd = local & 7;
   // selects of values: an indexed member would put the whole struct in scratch
   const int c0 = M.nch[0], c1 = M.nch[1], c2 = M.nch[2], c3 = M.nch[3];
@@ -169,9 +171,10 @@ __device__ __forceinline__ bool vxc_item(const VxcMol& M, int nsv, VxcItem& it) 
   }
   it.a0 = row * M.tb;
   it.b0 = col * M.tb;
-  it.rbeg = it.chunk * ch;
-  it.rend = min(M.npts_pad, it.rbeg + ch);
-  return true;
+  const int r0 = slab * M.slab, r1 = min(M.npts_pad, r0 + M.slab);
+  it.rbeg = r0 + it.chunk * ch;
+  it.rend = min(r1, it.rbeg + ch);
+  return it.rbeg < r1;   // a shorter last slab has fewer chunks
 }
 
 // Quadrant of this wave in a tile of tr x tc blocks: rows from wi, columns from wj, at most 2 x 2 blocks,
@@ -221,14 +224,17 @@ __device__ __forceinline__ float readlane_f32(float x, int lane) {
 // many issue slots as the products (28% MFMA, 50% VALU busy at n = 560): row addresses stay scalar, u
 // is a pair of FP32 numbers held one point a lane and read by lane index.
 constexpr int VX_FL = 2;
+// Z is formed and multiplied a slab of points at a time, whose sums add to the partials of the slab
+// before (the same chunks of every slab, one launch after the other: a fixed order).  vxc_slabs has
+// the sizes.
 
 __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __restrict__ mols, int nmol,
-                                                                const VxcMol one, int nsv) {
+                                                                const VxcMol one, int nsv, int slab) {
   __shared__ __align__(16) __bf16 Ls[3][4][VX_CP * 8];
   __shared__ __align__(16) __bf16 Rs[3][4][VX_CP * 8];
   const VxcMol M = vxc_find<&VxcMol::blk0>(mols, nmol, one, blockIdx.x);
   VxcItem it;
-  if (!vxc_item<float>(M, nsv, it)) return;
+  if (!vxc_item<float>(M, nsv, slab, it)) return;
   const bool sym = it.cls == 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r = lane & 15, nP = M.nP;
@@ -240,8 +246,10 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
   // repeat the last one (their blocks are not computed)
   const unsigned cl = 4 * min(it.a0 * 16 + lane, nP - 1), cr = 4 * min(it.b0 * 16 + lane, nP - 1);
   const gptr<float> lp = (gptr<float>)M.ao;
-  const gptr<float> rp = sym ? lp : (gptr<float>)M.z + it.s * plane;
-  const gptr<f2v> up = (gptr<f2v>)M.u + (size_t)it.s * M.npts_pad + (lane & 31);
+  const size_t r0 = (size_t)slab * M.slab;   // Z and u start with the slab
+  const gptr<float> rp = sym ? lp : (gptr<float>)M.z + (size_t)it.s * M.slab * nP;
+  const size_t rs = sym ? 0 : r0 * nP;
+  const gptr<f2v> up = (gptr<f2v>)M.u + (size_t)it.s * M.slab + (lane & 31);
   float xl[8], xr[8];
   f2v u = {0.f, 0.f};   // u of point lane % 32 of the loaded stage
   auto gload = [&](int pt, int pl) {
@@ -249,9 +257,9 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       xl[e] = row_load<float>(lp + row + e * nP, cl);
-      xr[e] = row_load<float>(rp + row + e * nP, cr);
+      xr[e] = row_load<float>(rp + (row - rs) + e * nP, cr);
     }
-    if (sym) u = up[pt];
+    if (sym) u = up[pt - r0];
   };
   auto lstore = [&]() {
     bf8 f[3];
@@ -322,8 +330,10 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
     for (int j = 0; j < 2; ++j)
       if (mask >> (i * 2 + j) & 1)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          out[(size_t)((it.a0 + wi + i) * 16 + mfma32_row(lane, v)) * nP + (it.b0 + wj + j) * 16 + r] = acc[i][j][v];
+        for (int v = 0; v < 4; ++v) {
+          const size_t at = (size_t)((it.a0 + wi + i) * 16 + mfma32_row(lane, v)) * nP + (it.b0 + wj + j) * 16 + r;
+          out[at] = slab ? out[at] + acc[i][j][v] : acc[i][j][v];
+        }
 }
 
 // FP64: an item is a pair of tiles (I, J), so that the planes of both are staged once for all five
@@ -464,7 +474,7 @@ __global__ __launch_bounds__(256, 2) inline void vxc_f64_kernel(const VxcMol* __
   __shared__ __align__(16) double Js[5][VXD_K][VXD_LD];   // tile J: phi, u d_j phi, Z
   const VxcMol M = vxc_find<&VxcMol::blk0>(mols, nmol, one, blockIdx.x);
   VxcItem it;
-  if (!vxc_item<double>(M, nsv, it)) return;
+  if (!vxc_item<double>(M, nsv, 0, it)) return;
   if (it.cls < 2) vxc_f64_item<true>(M, it, vpt, vpt_rows, nsv, Is, Js);
   else vxc_f64_item<false>(M, it, vpt, vpt_rows, nsv, Is, Js);
 }

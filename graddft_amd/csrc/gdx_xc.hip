@@ -620,17 +620,18 @@ constexpr int RED_GROUPS = 32; // slice groups of the first reduction stage
 std::mutex vxc_tune_mu;
 std::map<std::tuple<int, int, int, int, int>, int> vxc_tune;
 
-// Tiling and chunks of one molecule, with about `budget` work items an XCD (spins counted): every class
+// Tiling and chunks of one molecule in slabs of `slab` points, with about `budget` work items an XCD (spins counted): every class
 // of items starts with eight chunks, one an XCD, and the class whose items cost most gets eight more
 // while they fit; chunks are not under 128 points, below which the nP x nP partials outweigh the
 // products.  FP32 spreads the blocks evenly over the tiles, FP64 keeps full tiles and one ragged tile
 // (n = 96: 64 + 32, whose products divide over four waves; those of 48 + 48 do not).
 template <typename T>
-VxcMol vxc_plan(int Np, int nP, int nsv, double budget) {
+VxcMol vxc_plan(int Np, int nP, int nsv, int slab, double budget) {
   VxcMol M{};
   const int nblk = nP / 16;
   M.npts_pad = Np;
   M.nP = nP;
+  M.slab = slab;
   const int nt = (nblk + VX_TB - 1) / VX_TB;
   M.tb = sizeof(T) == 4 ? (nblk + nt - 1) / nt : std::min(nblk, VX_TB);
   M.nf = nblk / M.tb;
@@ -647,13 +648,13 @@ VxcMol vxc_plan(int Np, int nP, int nsv, double budget) {
     for (int c = 0; c < 4; ++c)
       if (tiles[c] && (top < 0 || vxc_cost<T>(M, c) * k[top] > vxc_cost<T>(M, top) * k[c])) top = c;
     used += tiles[top] * nsv;
-    if (used > budget || (k[top] + 1) * 8 * 128 > Np) break;
+    if (used > budget || (k[top] + 1) * 8 * 128 > slab) break;
     ++k[top];
   }
   for (int c = 0; c < 4; ++c) {
     if (!tiles[c]) continue;
-    M.ch[c] = ((Np + 8 * k[c] - 1) / (8 * k[c]) + VX_PTS - 1) / VX_PTS * VX_PTS;
-    M.nch[c] = (Np + M.ch[c] - 1) / M.ch[c];
+    M.ch[c] = ((slab + 8 * k[c] - 1) / (8 * k[c]) + VX_PTS - 1) / VX_PTS * VX_PTS;
+    M.nch[c] = (slab + M.ch[c] - 1) / M.ch[c];
   }
   return M;
 }
@@ -663,16 +664,29 @@ inline double vxc_work(int Np, int nP) {   // block products of one spin
 }
 // resident blocks an XCD: four a CU (FP32), two (FP64)
 inline int vxc_slots(bool fp64) { return NUM_CU / 8 * (fp64 ? 2 : 4); }
-// FP32 scratch of both spins: Z of `el` AO elements and u pairs of `rows` points
-inline size_t vxc_z_bytes(size_t el, size_t rows) { return 2 * (el * 4 + rows * 8); }
+// FP32 scratch: Z of `el` AO elements and u pairs of `rows` points a spin
+inline size_t vxc_z_bytes(size_t el, size_t rows, int nsv) { return nsv * (el * 4 + rows * 8); }
+// FP32: slabs of points, so that their Z takes no more than the MLP deltas over which it lies, or than
+// ZCAP (zbytes gives the scratch for a number of slabs).  Z of the whole grid was 2.0 GB at n = 560, 427k
+// points; V_xc of both spins takes 13.3 ms there with it, 11.8 in slabs of 128 MB (they stay in the
+// last-level cache), and level within 1% at n = 82 .. 280; slabs of 64 MB cost 5 to 9% at n = 102 .. 280.
+constexpr size_t ZCAP = (size_t)128 << 20;
+inline int vxc_slab(int Np, int nslab) { return ((Np + nslab - 1) / nslab + 63) / 64 * 64; }
+template <typename F>
+int vxc_slabs(const F& zbytes, size_t gbytes) {
+  const size_t cap = std::max(gbytes, ZCAP);
+  int n = (int)((zbytes(1) + cap - 1) / cap);
+  while (zbytes(n) > cap && zbytes(n + 1) < zbytes(n)) ++n;
+  return n;
+}
 // one molecule: one round of resident blocks, or as many as give each class two chunks an XCD
 template <typename T>
-VxcMol vxc_single(int Np, int nP, int nsv) {
-  const int slots = vxc_slots(sizeof(T) == 8);
-  const VxcMol M = vxc_plan<T>(Np, nP, nsv, 0);
+VxcMol vxc_single(int Np, int nP, int nsv, int nslab) {
+  const int slots = vxc_slots(sizeof(T) == 8), slab = vxc_slab(Np, nslab);
+  const VxcMol M = vxc_plan<T>(Np, nP, nsv, slab, 0);
   int items = 0;
   for (int c = 0; c < 4; ++c) items += 2 * vxc_tiles<T>(M, c) * nsv;
-  return vxc_plan<T>(Np, nP, nsv, (items + slots - 1) / slots * slots);
+  return vxc_plan<T>(Np, nP, nsv, slab, (items + slots - 1) / slots * slots);
 }
 constexpr int SKW_ROWS = 512;  // grid points per block of the skinny weight-gradient kernel
 
@@ -684,7 +698,7 @@ struct Layout {
   size_t Dp2, dpart_t, dfin_t, Edot, ZT, GEd, edot_part, scal, rtmp;
   size_t total;
   size_t hstride;  // elements between the activation buffers of consecutive layers
-  int nsd, nchunk, nsplit, kchunk, kseg, sps, npt_blocks, nwblk, wrows, rows;
+  int nsd, nchunk, nslab, nsplit, kchunk, kseg, sps, npt_blocks, nwblk, wrows, rows;
   size_t nparam;
 };
 
@@ -699,10 +713,17 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   const int hmode = d.kind == GDX_FUNC_B3LYP_NEURAL_CORR ? 1 : 0;
   L.nsd = d.spin_restricted ? 1 : 2;
   L.rows = (int)R;
+  const int nsv_max = hvp || neural || !d.spin_restricted ? 2 : 1;   // spins of V_xc builds
+  L.Gbytes = neural ? 2 * R * d.mlp_h * es : 0;
+  auto zbytes = [&](int nslab) {
+    const size_t slab = vxc_slab((int)Np, nslab);
+    return vxc_z_bytes(slab * nP, slab, nsv_max);
+  };
+  L.nslab = batch || es == 8 ? 1 : vxc_slabs(zbytes, L.Gbytes);
   L.nchunk = 0;   // V_xc partial slots (chunks x nsv)
-  for (int nsv : {1, 2})
-    L.nchunk = std::max<int>(L.nchunk, nsv * (es == 8 ? vxc_part_slots<double>(vxc_single<double>((int)Np, (int)nP, nsv))
-                                                      : vxc_part_slots<float>(vxc_single<float>((int)Np, (int)nP, nsv))));
+  for (int nsv = 1; nsv <= nsv_max; ++nsv)
+    L.nchunk = std::max<int>(L.nchunk, nsv * (es == 8 ? vxc_part_slots<double>(vxc_single<double>((int)Np, (int)nP, nsv, 1))
+                                                      : vxc_part_slots<float>(vxc_single<float>((int)Np, (int)nP, nsv, L.nslab))));
   // split-K for the hidden weight-gradient GEMMs: 128 splits of whole 32-row stages, the
   // last one of a segment shorter; for hvp the value and tangent rows are two segments of
   // 64 splits each, so the first half of the splits covers the value rows exactly
@@ -751,11 +772,10 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   L.DX = take(neural ? R * d.mlp_nc * es : 0);
   L.vpt = take(2 * Np * VPT_STRIDE * 8);
   L.vpart = take(batch ? 0 : (size_t)L.nchunk * nP * nP * 8);
-  // FP32: Z, then the pairs of u, over the MLP deltas where they are large enough (the V_xc build comes
-  // after the last use of G)
-  const size_t zbytes = batch || es == 8 ? 0 : vxc_z_bytes(Np * nP, Np);
-  L.Gbytes = neural ? 2 * R * h * es : 0;
-  L.Z = zbytes <= L.Gbytes ? L.G : take(zbytes);
+  // FP32: Z, then the pairs of u, of a slab, over the MLP deltas where they are large enough (the V_xc
+  // build comes after the last use of G)
+  const size_t zslab = batch || es == 8 ? 0 : zbytes(L.nslab);
+  L.Z = zslab <= L.Gbytes ? L.G : take(zslab);
   size_t wbytes = 0;
   if (neural) {
     wbytes = (size_t)L.nsplit * h * h * es;
@@ -766,7 +786,7 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   L.wpart = take(wbytes);
   L.cpart = take(neural ? (size_t)L.nsplit * h * es : 0);
   // two-stage reductions: up to two at once (reduce_slices2: the largest one plus the last layer's bias)
-  L.rtmp = take((size_t)RED_GROUPS * (std::max(std::max(h * h, 16 * h), 2 * nP * nP) + 64) * 8);
+  L.rtmp = take((size_t)RED_GROUPS * (std::max(h * h, 16 * h) + 64) * 8);
   if (hvp) {
     L.Dp2 = take(batch ? 0 : dpack);
     L.dpart_t = take(2 * Np * DENS_STRIDE * 8);
@@ -948,7 +968,7 @@ struct BatchCtx {
   // V_xc (tiles of 64): the molecules' tables for one and for two spins' potentials
   struct Vxc {
     const VxcMol* d_mols = nullptr;
-    int blocks = 0, zblocks = 0, rblocks = 0;
+    int blocks = 0, zblocks = 0, nslab = 1, rblocks = 0;
   } vx[2];
   const int* seg256 = nullptr;               // (nmol + 1) segment starts in 256-row blocks
   const int* seg64 = nullptr;                // in 64-row blocks
@@ -1009,14 +1029,16 @@ void launch_density(const Ctx& c, const T* ao, const double* mats, bool tangent,
 // V_xc products of one molecule (`one`, mols null) or a batch, reduced into d_rdm1
 template <typename T>
 void launch_vxc_kernels(const Ctx& c, const VxcMol* mols, int nmol, const VxcMol& one, int blocks, int zblocks,
-                        int rblocks, int nsv, double* d_rdm1) {
+                        int nslab, int rblocks, int nsv, double* d_rdm1) {
   hipStream_t st = c.st;
   const char* nm = gname<T>(c.d, "vxc_f64", "vxc_f32", "vxc_bf16x6");
   const double* vpt = c.P<double>(c.L.vpt);
   const size_t rows = (size_t)c.d.npts_pad;
   if constexpr (sizeof(T) == 4) {
-    GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(zblocks), dim3(NT), 0, st, mols, nmol, one, vpt, rows, nsv);
-    GDX_LAUNCH(nm, vxc_f32_kernel, dim3(blocks), dim3(NT), 0, st, mols, nmol, one, nsv);
+    for (int slab = 0; slab < nslab; ++slab) {
+      GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(zblocks), dim3(NT), 0, st, mols, nmol, one, vpt, rows, nsv, slab);
+      GDX_LAUNCH(nm, vxc_f32_kernel, dim3(blocks), dim3(NT), 0, st, mols, nmol, one, nsv, slab);
+    }
   } else {
     GDX_LAUNCH(nm, vxc_f64_kernel, dim3(blocks), dim3(NT), 0, st, mols, nmol, one, vpt, rows, nsv);
   }
@@ -1026,7 +1048,7 @@ void launch_vxc_kernels(const Ctx& c, const VxcMol* mols, int nmol, const VxcMol
 template <typename T>
 void launch_vxc_batch(const Ctx& c, int nsv, double* d_rdm1) {
   const BatchCtx::Vxc& V = c.b->vx[nsv - 1];
-  launch_vxc_kernels<T>(c, V.d_mols, c.b->nmol, VxcMol{}, V.blocks, V.zblocks, V.rblocks, nsv, d_rdm1);
+  launch_vxc_kernels<T>(c, V.d_mols, c.b->nmol, VxcMol{}, V.blocks, V.zblocks, V.nslab, V.rblocks, nsv, d_rdm1);
 }
 
 // densities: fragments of D -> density -> point_fwd
@@ -1143,13 +1165,13 @@ void reduce_slices2(const Ctx& c, const TP* p0, int ns0, long st0, long len0, do
 template <typename T>
 void launch_vxc(const Ctx& c, const T* ao, int nsv, double* d_rdm1) {
   const gdx_xc_desc& d = c.d;
-  VxcMol M = vxc_single<T>(d.npts_pad, d.nao_pad, nsv);
+  VxcMol M = vxc_single<T>(d.npts_pad, d.nao_pad, nsv, c.L.nslab);
   M.ao = ao;
   M.z = c.P<float>(c.L.Z);
-  M.u = M.z + 2 * (size_t)d.npts_pad * d.nao_pad;
+  M.u = M.z + (size_t)nsv * M.slab * d.nao_pad;
   M.part = c.P<double>(c.L.vpart);
   M.n = d.nao;
-  launch_vxc_kernels<T>(c, nullptr, 1, M, vxc_blocks<T>(M, nsv), (int)((size_t)d.npts_pad * d.nao_pad / 1024),
+  launch_vxc_kernels<T>(c, nullptr, 1, M, vxc_blocks<T>(M, nsv), (int)((size_t)M.slab * d.nao_pad / 1024), c.L.nslab,
                         (int)vxc_reduce_blocks(M, nsv), nsv, d_rdm1);
 }
 
@@ -1625,6 +1647,16 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
   // level 1, FP64: chunks of a fixed 2048 points were 40-66 blocks a launch)
   double batch_work = 0.0;
   for (int m = 0; m < nmol; ++m) batch_work += vxc_work(mols[m].npts_pad, mols[m].nao_pad);
+  auto zall = [&](int nslab) {
+    size_t z = 0;
+    for (int m = 0; m < nmol; ++m) {
+      const size_t slab = vxc_slab(mols[m].npts_pad, nslab);
+      z += vxc_z_bytes(slab * mols[m].nao_pad, slab, 2);
+    }
+    return z;
+  };
+  const Layout& Lz = P->hvp ? P->Lh : P->L;   // as in make_layout: over the MLP deltas where they fit
+  const int nslab = es == 8 ? 1 : vxc_slabs(zall, Lz.Gbytes);
   for (int m = 0; m < nmol; ++m) {
     const gdx_xc_batch_mol& M = mols[m];
     const int nP = M.nao_pad, n = M.nao;
@@ -1654,7 +1686,8 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     for (int nsv = 1; nsv <= nsv_max; ++nsv) {
       // four rounds of resident blocks: the items of different molecules are not alike
       const double budget = 4 * vxc_slots(es == 8) * vxc_work(M.npts_pad, nP) / batch_work;
-      VxcMol v = es == 8 ? vxc_plan<double>(M.npts_pad, nP, nsv, budget) : vxc_plan<float>(M.npts_pad, nP, nsv, budget);
+      VxcMol v = es == 8 ? vxc_plan<double>(M.npts_pad, nP, nsv, M.npts_pad, budget)
+                         : vxc_plan<float>(M.npts_pad, nP, nsv, vxc_slab(M.npts_pad, nslab), budget);
       v.ao = M.ao;
       v.row0 = row;
       v.n = n;
@@ -1666,7 +1699,7 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     dm += 2L * n * n;
     dp += 2 * (es == 8 ? dens_pack_bytes<double>(nP) : dens_pack_bytes<float>(nP));
     vp += slots * nP * nP;
-    zel += 2L * M.npts_pad * nP;
+    zel += (long)vxc_z_bytes((size_t)vxc_slab(M.npts_pad, nslab) * nP, vxc_slab(M.npts_pad, nslab), 2) / 4;
   }
   seg256[nmol] = (int)(row / 256);
   seg64[nmol] = (int)(row / 64);
@@ -1682,8 +1715,7 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
   const size_t o_w = take(rows * 8), o_wg = take(rows * 8), o_gpt = take(rows * 8);
   const size_t o_one = take(8), o_scal = take(nmol * 8);
   const size_t o_dp = take(dp), o_dpt = take(P->hvp ? dp : 0);
-  const size_t o_vp = take(vp * 8), zbytes = es == 4 ? vxc_z_bytes(zel / 2, rows) : 0;   // (FP64 items form Z themselves)
-  const Layout& Lz = P->hvp ? P->Lh : P->L;   // as in make_layout: over the MLP deltas where they fit
+  const size_t o_vp = take(vp * 8), zbytes = es == 4 ? zel * 4 : 0;   // (FP64 items form Z themselves)
   const bool z_in_g = zbytes <= Lz.Gbytes;
   const size_t o_z = take(z_in_g ? 0 : zbytes);
   auto fail = [&](hipError_t e, const char* what) {
@@ -1706,7 +1738,7 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     for (int k = 0; k < 2; ++k) {
       vmol[k][m].part = (double*)(T0 + o_vp) + vpart_off[m];
       vmol[k][m].z = (float*)Z0 + z_off[m];
-      vmol[k][m].u = (float*)Z0 + zel + 4 * (size_t)rowv[m];   // both spins' pairs of this molecule's rows
+      vmol[k][m].u = vmol[k][m].z + 2 * (size_t)vmol[k][m].slab * vmol[k][m].nP;
     }
   }
   for (int k = 0; k < 2; ++k) {
@@ -1717,10 +1749,11 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
       v.zblk0 = V.zblocks;
       v.rblk0 = V.rblocks;
       V.blocks += es == 8 ? vxc_blocks<double>(v, k + 1) : vxc_blocks<float>(v, k + 1);
-      V.zblocks += (int)((long)v.npts_pad * v.nP / 1024);
+      V.zblocks += (int)((long)v.slab * v.nP / 1024);
       V.rblocks += (int)vxc_reduce_blocks(v, k + 1);
     }
     V.d_mols = (const VxcMol*)(T0 + o_vm[k]);
+    V.nslab = nslab;
   }
   const double one = 1.0;
   struct Up { size_t off; const void* src; size_t bytes; };

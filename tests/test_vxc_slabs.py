@@ -1,0 +1,98 @@
+"""The FP32 V_xc build forms its operand Z a slab of grid points at a time in a scratch of bounded size:
+the workspace does not grow with points x basis functions, and the slabs' sums are those of the grid."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+
+def _workspace(n, npts, precision, h=0, hvp=False):
+    from graddft_amd import _lib
+    d = _lib.XCDesc()
+    d.npts = d.npts_pad = npts
+    d.nao, d.nao_pad = n, (n + 15) // 16 * 16
+    d.precision = precision
+    d.spin_restricted = 0
+    if h:
+        d.kind, d.mlp_nc, d.mlp_h, d.mlp_nhidden, d.mlp_nd = _lib.GDX_FUNC_NEURAL_B3LYP, 6, h, 3, 4
+    size = ctypes.c_size_t(0)
+    lib = _lib.load()
+    call = lib.gdx_xc_hvp_workspace_size if hvp else lib.gdx_xc_workspace_size
+    _lib.check(call(ctypes.byref(d), ctypes.byref(size)), "workspace size")
+    return size.value
+
+
+@pytest.mark.parametrize("hvp", [False, True])
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("h", [0, 32, 128, 256])
+def test_workspace_does_not_grow_with_points_times_functions(h, precision, hvp):
+    def basis_part(n, npts):
+        return _workspace(n, npts, precision, h, hvp) - _workspace(16, npts, precision, h, hvp)
+    # what a point keeps (densities, energies, potentials, activations) has no basis functions in it; the
+    # scratch for Z is 128 MiB at most, or lies over the network's deltas
+    for n in (300, 560, 1100):
+        assert basis_part(n, 1_600_000) - basis_part(n, 400_000) <= 128 << 20
+
+
+def _molecule(n, npts, seed):
+    from graddft_amd.molecule import Grid, Molecule
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rows, cols = (npts + 255) // 256 * 256, (n + 15) // 16 * 16
+    planes = torch.zeros((5, rows, cols), dtype=torch.float64, device="cuda")
+    for k in range(5):
+        planes[k, :npts, :n] = torch.randn((npts, n), dtype=torch.float64, device="cuda", generator=g) / np.sqrt(n)
+    w = torch.zeros(rows, dtype=torch.float64, device="cuda")
+    w[:npts] = torch.rand(npts, dtype=torch.float64, device="cuda", generator=g) + 0.1
+    c = torch.randn((2, n, max(2, n // 3)), dtype=torch.float64, device="cuda", generator=g)
+    z = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    return Molecule(grid=Grid(torch.zeros((npts, 3), dtype=torch.float64, device="cuda"), w[:npts], w),
+                    atom_index=torch.ones(1), nuclear_pos=torch.zeros((1, 3)), ao_planes=planes,
+                    rdm1=0.3 * c @ c.transpose(1, 2), nuclear_repulsion=0.0, h1e=z, s1e=z,
+                    mo_coeff=torch.zeros((2, n, n)), mo_occ=torch.zeros((2, n)), mo_energy=torch.zeros((2, n)),
+                    restricted=False)
+
+
+def _rel(a, b):
+    return float((a - b).norm() / b.norm())
+
+
+# sums over 1e5 points of products rounded by 2^-24 each, no cancellation: 2e-7 expected
+TOL = 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,npts", [(330, 60000), (209, 82000)])
+def test_single_molecule(n, npts):
+    from graddft_amd import B3LYP_GRID, XCEnergyVxcFn
+    m = _molecule(n, npts, n)
+    print(f"case: slabs, n={n} npts={npts}, Z {8e-6 * m.nao_pad * m.npts_pad:.0f} MB", flush=True)
+    out = {}
+    for restricted in (False, True):
+        mm = m.replace(restricted=restricted, rdm1=torch.stack([m.rdm1[0]] * 2) if restricted else m.rdm1)
+        for p in ("fp64", "fp32"):
+            D = mm.rdm1.detach().requires_grad_(True)
+            E, V = XCEnergyVxcFn.apply(D, None, B3LYP_GRID.plan(mm, p))
+            out[p] = (V.detach(), *torch.autograd.grad([E, V], [D], [torch.ones_like(E), D.detach()]))
+        for a, b in zip(out["fp32"], out["fp64"]):
+            assert _rel(a, b) <= TOL
+
+
+@pytest.mark.gpu
+def test_batch_with_a_molecule_shorter_than_the_slabs():
+    from graddft_amd import B3LYP_GRID
+    from graddft_amd.batch import XCBatchPlan
+    mols = [_molecule(330, 70000, 1), _molecule(20, 200, 2), _molecule(209, 90000, 3)]
+    print("case: batch in slabs, one molecule with empty last slabs", flush=True)
+    out = {}
+    for p in ("fp64", "fp32"):
+        plan = XCBatchPlan(B3LYP_GRID, mols, p, restricted=False, hvp=False)
+        D = plan.concat([m.rdm1 for m in mols])
+        e = torch.empty(3, dtype=torch.float64, device="cuda")
+        dD = torch.empty_like(D)
+        plan.forward(D, None, e)
+        plan.backward(None, torch.ones_like(e), dD, None)
+        out[p] = [v.clone() for v in plan.split(dD)]
+        plan.close()
+    for a, b in zip(out["fp32"], out["fp64"]):
+        assert _rel(a, b) <= TOL
