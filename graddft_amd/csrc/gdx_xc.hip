@@ -658,10 +658,6 @@ VxcMol vxc_plan(int Np, int nP, int nsv, int slab, double budget) {
   }
   return M;
 }
-inline double vxc_work(int Np, int nP) {   // block products of one spin
-  const double nblk = nP / 16;
-  return Np * (nblk * nblk + 1.5 * nblk * (nblk + 1));
-}
 // resident blocks an XCD: four a CU (FP32), two (FP64)
 inline int vxc_slots(bool fp64) { return NUM_CU / 8 * (fp64 ? 2 : 4); }
 // FP32 scratch: Z of `el` AO elements and u pairs of `rows` points a spin
@@ -688,6 +684,11 @@ VxcMol vxc_single(int Np, int nP, int nsv, int nslab) {
   for (int c = 0; c < 4; ++c) items += 2 * vxc_tiles<T>(M, c) * nsv;
   return vxc_plan<T>(Np, nP, nsv, slab, (items + slots - 1) / slots * slots);
 }
+// a molecule of a batch: by itself, so that its sums do not depend on the molecules beside it; enough
+// items that three small molecules fill the card, not so many that the partials of many weigh (against
+// four rounds shared by the batch: alkanes C1-C3, level 1, FP64 238 -> 245 us and 128 -> 71 MB of plan;
+// 24 of C1-C4 2.21 -> 1.96 ms, 432 -> 644 MB; C1-C8, level 2, FP32 neural 3.79 -> 3.57 ms)
+inline double vxc_batch_budget(bool fp64) { return vxc_slots(fp64) * (fp64 ? 0.5 : 0.75); }
 constexpr int SKW_ROWS = 512;  // grid points per block of the skinny weight-gradient kernel
 
 // hvp = true: activation-side buffers hold stacked [value; tangent] rows (R = 2 N_pad), plus
@@ -965,10 +966,15 @@ struct BatchCtx {
     const DensMol* d_mols = nullptr;
     int blocks = 0, pblocks = 0;
   } dn[3];
-  // V_xc (tiles of 64): the molecules' tables for one and for two spins' potentials
+  // V_xc (tiles of 64): the molecules' tables for one and for two spins' potentials, and the groups of
+  // consecutive molecules that share a launch and, in FP32, the scratch for Z
+  struct Group {
+    int first = 0, nmol = 0, blocks = 0, zblocks = 0, nslab = 1;
+  };
   struct Vxc {
     const VxcMol* d_mols = nullptr;
-    int blocks = 0, zblocks = 0, nslab = 1, rblocks = 0;
+    std::vector<Group> groups;
+    int rblocks = 0;
   } vx[2];
   const int* seg256 = nullptr;               // (nmol + 1) segment starts in 256-row blocks
   const int* seg64 = nullptr;                // in 64-row blocks
@@ -1026,29 +1032,29 @@ void launch_density(const Ctx& c, const T* ao, const double* mats, bool tangent,
              out);
 }
 
-// V_xc products of one molecule (`one`, mols null) or a batch, reduced into d_rdm1
+// V_xc products of one molecule (`one`, mols null) or a group of a batch's
 template <typename T>
-void launch_vxc_kernels(const Ctx& c, const VxcMol* mols, int nmol, const VxcMol& one, int blocks, int zblocks,
-                        int nslab, int rblocks, int nsv, double* d_rdm1) {
+void launch_vxc_group(const Ctx& c, const VxcMol* mols, const VxcMol& one, const BatchCtx::Group& G, int nsv) {
   hipStream_t st = c.st;
   const char* nm = gname<T>(c.d, "vxc_f64", "vxc_f32", "vxc_bf16x6");
   const double* vpt = c.P<double>(c.L.vpt);
   const size_t rows = (size_t)c.d.npts_pad;
   if constexpr (sizeof(T) == 4) {
-    for (int slab = 0; slab < nslab; ++slab) {
-      GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(zblocks), dim3(NT), 0, st, mols, nmol, one, vpt, rows, nsv, slab);
-      GDX_LAUNCH(nm, vxc_f32_kernel, dim3(blocks), dim3(NT), 0, st, mols, nmol, one, nsv, slab);
+    for (int slab = 0; slab < G.nslab; ++slab) {
+      GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(G.zblocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
+      GDX_LAUNCH(nm, vxc_f32_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, nsv, slab);
     }
   } else {
-    GDX_LAUNCH(nm, vxc_f64_kernel, dim3(blocks), dim3(NT), 0, st, mols, nmol, one, vpt, rows, nsv);
+    GDX_LAUNCH(nm, vxc_f64_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv);
   }
-  GDX_LAUNCH("reduce_vxc", vxc_reduce_kernel<T>, dim3(rblocks), dim3(NT), 0, st, mols, nmol, one, nsv, d_rdm1);
 }
 
 template <typename T>
 void launch_vxc_batch(const Ctx& c, int nsv, double* d_rdm1) {
   const BatchCtx::Vxc& V = c.b->vx[nsv - 1];
-  launch_vxc_kernels<T>(c, V.d_mols, c.b->nmol, VxcMol{}, V.blocks, V.zblocks, V.nslab, V.rblocks, nsv, d_rdm1);
+  for (const BatchCtx::Group& G : V.groups) launch_vxc_group<T>(c, V.d_mols + G.first, VxcMol{}, G, nsv);
+  GDX_LAUNCH("reduce_vxc", vxc_reduce_kernel<T>, dim3(V.rblocks), dim3(NT), 0, c.st, V.d_mols, c.b->nmol, VxcMol{}, nsv,
+             d_rdm1);
 }
 
 // densities: fragments of D -> density -> point_fwd
@@ -1171,8 +1177,14 @@ void launch_vxc(const Ctx& c, const T* ao, int nsv, double* d_rdm1) {
   M.u = M.z + (size_t)nsv * M.slab * d.nao_pad;
   M.part = c.P<double>(c.L.vpart);
   M.n = d.nao;
-  launch_vxc_kernels<T>(c, nullptr, 1, M, vxc_blocks<T>(M, nsv), (int)((size_t)M.slab * d.nao_pad / 1024), c.L.nslab,
-                        (int)vxc_reduce_blocks(M, nsv), nsv, d_rdm1);
+  BatchCtx::Group G;
+  G.nmol = 1;
+  G.blocks = vxc_blocks<T>(M, nsv);
+  G.zblocks = (int)((size_t)M.slab * d.nao_pad / 1024);
+  G.nslab = c.L.nslab;
+  launch_vxc_group<T>(c, nullptr, M, G, nsv);
+  GDX_LAUNCH("reduce_vxc", vxc_reduce_kernel<T>, dim3((int)vxc_reduce_blocks(M, nsv)), dim3(NT), 0, c.st, nullptr, 1, M,
+             nsv, d_rdm1);
 }
 
 template <typename T>
@@ -1640,23 +1652,21 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
   std::vector<size_t> pack_off(nmol);
   std::vector<VxcMol> vmol[2];            // [nsv - 1][molecule]
   std::vector<int> seg256(nmol + 1), seg64(nmol + 1), rowv(nmol + 1);
-  long row = 0, dm = 0, dp = 0, vp = 0, zel = 0;
+  long row = 0, dm = 0, dp = 0, vp = 0;
   P->dm_off.resize(nmol + 1);
-  std::vector<long> vpart_off(nmol), z_off(nmol);
-  // V_xc: one launch, whose items should fill the CUs several times over (three alkanes C1-C3,
-  // level 1, FP64: chunks of a fixed 2048 points were 40-66 blocks a launch)
-  double batch_work = 0.0;
-  for (int m = 0; m < nmol; ++m) batch_work += vxc_work(mols[m].npts_pad, mols[m].nao_pad);
-  auto zall = [&](int nslab) {
-    size_t z = 0;
-    for (int m = 0; m < nmol; ++m) {
-      const size_t slab = vxc_slab(mols[m].npts_pad, nslab);
-      z += vxc_z_bytes(slab * mols[m].nao_pad, slab, 2);
-    }
-    return z;
-  };
-  const Layout& Lz = P->hvp ? P->Lh : P->L;   // as in make_layout: over the MLP deltas where they fit
-  const int nslab = es == 8 ? 1 : vxc_slabs(zall, Lz.Gbytes);
+  std::vector<long> vpart_off(nmol);
+  // V_xc: chunks and slabs of a molecule by itself, whatever its neighbours, so that its sums are the
+  // same in every batch.  FP32: Z of a group of molecules in the scratch that make_layout's rule gives
+  // the whole batch, over the MLP deltas where those are larger
+  const Layout& Lz = P->hvp ? P->Lh : P->L;
+  std::vector<int> nslab(nmol, 1);
+  std::vector<size_t> zbytes_of(nmol, 0);
+  for (int m = 0; m < nmol && es == 4; ++m) {
+    const int Np = mols[m].npts_pad, nP = mols[m].nao_pad;
+    auto zbytes = [&](int k) { return vxc_z_bytes((size_t)vxc_slab(Np, k) * nP, vxc_slab(Np, k), 2); };
+    nslab[m] = vxc_slabs(zbytes, is_neural(d) ? 2 * (size_t)Np * d.mlp_h * es : 0);
+    zbytes_of[m] = zbytes(nslab[m]);
+  }
   for (int m = 0; m < nmol; ++m) {
     const gdx_xc_batch_mol& M = mols[m];
     const int nP = M.nao_pad, n = M.nao;
@@ -1681,13 +1691,11 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
           (int)(((es == 8 ? dens_pack_threads<double>(nP, nspin) : dens_pack_threads<float>(nP, nspin)) + 255) / 256);
     }
     vpart_off[m] = vp;
-    z_off[m] = zel;
     long slots = 0;
     for (int nsv = 1; nsv <= nsv_max; ++nsv) {
-      // four rounds of resident blocks: the items of different molecules are not alike
-      const double budget = 4 * vxc_slots(es == 8) * vxc_work(M.npts_pad, nP) / batch_work;
+      const double budget = vxc_batch_budget(es == 8);
       VxcMol v = es == 8 ? vxc_plan<double>(M.npts_pad, nP, nsv, M.npts_pad, budget)
-                         : vxc_plan<float>(M.npts_pad, nP, nsv, vxc_slab(M.npts_pad, nslab), budget);
+                         : vxc_plan<float>(M.npts_pad, nP, nsv, vxc_slab(M.npts_pad, nslab[m]), budget);
       v.ao = M.ao;
       v.row0 = row;
       v.n = n;
@@ -1699,7 +1707,6 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     dm += 2L * n * n;
     dp += 2 * (es == 8 ? dens_pack_bytes<double>(nP) : dens_pack_bytes<float>(nP));
     vp += slots * nP * nP;
-    zel += (long)vxc_z_bytes((size_t)vxc_slab(M.npts_pad, nslab) * nP, vxc_slab(M.npts_pad, nslab), 2) / 4;
   }
   seg256[nmol] = (int)(row / 256);
   seg64[nmol] = (int)(row / 64);
@@ -1715,9 +1722,32 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
   const size_t o_w = take(rows * 8), o_wg = take(rows * 8), o_gpt = take(rows * 8);
   const size_t o_one = take(8), o_scal = take(nmol * 8);
   const size_t o_dp = take(dp), o_dpt = take(P->hvp ? dp : 0);
-  const size_t o_vp = take(vp * 8), zbytes = es == 4 ? zel * 4 : 0;   // (FP64 items form Z themselves)
-  const bool z_in_g = zbytes <= Lz.Gbytes;
-  const size_t o_z = take(z_in_g ? 0 : zbytes);
+  const size_t o_vp = take(vp * 8), zcap = std::max(Lz.Gbytes, 2 * ZCAP);
+  // V_xc tables in falling order of a molecule's work, so that a launch ends with its shortest items, in
+  // groups whose Z fits (a molecule's own does, but for rounding: then it is a group and the scratch)
+  std::vector<int> order(nmol);
+  for (int m = 0; m < nmol; ++m) order[m] = m;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return (long)mols[a].npts_pad * mols[a].nao_pad * mols[a].nao_pad > (long)mols[b].npts_pad * mols[b].nao_pad * mols[b].nao_pad;
+  });
+  std::vector<BatchCtx::Group> groups;
+  std::vector<size_t> z_off(nmol, 0);
+  size_t zscratch = 0, zused = 0;
+  for (int i = 0; i < nmol; ++i) {
+    const int m = order[i];
+    if (i == 0 || zused + zbytes_of[m] > zcap) {
+      groups.emplace_back();
+      groups.back().first = i;
+      zused = 0;
+    }
+    z_off[m] = zused;
+    zused += round_up(zbytes_of[m], 256);
+    zscratch = std::max(zscratch, zused);
+    groups.back().nmol++;
+    groups.back().nslab = std::max(groups.back().nslab, nslab[m]);
+  }
+  const bool z_in_g = zscratch <= Lz.Gbytes;
+  const size_t o_z = take(z_in_g ? 0 : zscratch);
   auto fail = [&](hipError_t e, const char* what) {
     set_error(std::string("gdx_xc_batch_create: ") + what + ": " + hipGetErrorString(e));
     batch_free(P);
@@ -1737,23 +1767,27 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     for (int k = 0; k < 3; ++k) dmol[k][m].pack = T0 + (k == 2 ? o_dpt : o_dp) + pack_off[m];
     for (int k = 0; k < 2; ++k) {
       vmol[k][m].part = (double*)(T0 + o_vp) + vpart_off[m];
-      vmol[k][m].z = (float*)Z0 + z_off[m];
+      vmol[k][m].z = (float*)(Z0 + z_off[m]);
       vmol[k][m].u = vmol[k][m].z + 2 * (size_t)vmol[k][m].slab * vmol[k][m].nP;
     }
   }
   for (int k = 0; k < 2; ++k) {
     BatchCtx::Vxc& V = P->B.vx[k];
-    for (int m = 0; m < nmol; ++m) {
-      VxcMol& v = vmol[k][m];
-      v.blk0 = V.blocks;
-      v.zblk0 = V.zblocks;
-      v.rblk0 = V.rblocks;
-      V.blocks += es == 8 ? vxc_blocks<double>(v, k + 1) : vxc_blocks<float>(v, k + 1);
-      V.zblocks += (int)((long)v.slab * v.nP / 1024);
-      V.rblocks += (int)vxc_reduce_blocks(v, k + 1);
-    }
     V.d_mols = (const VxcMol*)(T0 + o_vm[k]);
-    V.nslab = nslab;
+    V.groups = groups;
+    std::vector<VxcMol> table;
+    for (int m : order) table.push_back(vmol[k][m]);
+    vmol[k] = table;
+    for (BatchCtx::Group& G : V.groups)
+      for (int m = G.first; m < G.first + G.nmol; ++m) {
+        VxcMol& v = vmol[k][m];
+        v.blk0 = G.blocks;
+        v.zblk0 = G.zblocks;
+        v.rblk0 = V.rblocks;
+        G.blocks += es == 8 ? vxc_blocks<double>(v, k + 1) : vxc_blocks<float>(v, k + 1);
+        G.zblocks += (int)((long)v.slab * v.nP / 1024);
+        V.rblocks += (int)vxc_reduce_blocks(v, k + 1);
+      }
   }
   const double one = 1.0;
   struct Up { size_t off; const void* src; size_t bytes; };

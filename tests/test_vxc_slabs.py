@@ -96,3 +96,35 @@ def test_batch_with_a_molecule_shorter_than_the_slabs():
         plan.close()
     for a, b in zip(out["fp32"], out["fp64"]):
         assert _rel(a, b) <= TOL
+
+
+def _batch_vxc(mols, pick, precision, functional, theta):
+    """(V, second-order dD) of molecule `pick` of a batch of these molecules."""
+    from graddft_amd.batch import XCBatchPlan
+    plan = XCBatchPlan(functional, mols, precision, restricted=False, hvp=True)
+    D = plan.concat([m.rdm1 for m in mols])
+    e = torch.empty(len(mols), dtype=torch.float64, device="cuda")
+    one = torch.ones_like(e)
+    V, H = torch.empty_like(D), torch.empty_like(D)
+    plan.forward(D, theta, e)
+    plan.backward(theta, one, V, None)
+    plan.hvp(D, theta, D, one, d_rdm1=H)
+    out = plan.split(V)[pick].clone(), plan.split(H)[pick].clone()
+    plan.close()
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_a_molecule_is_the_same_in_every_batch(precision):
+    """Bit for bit: its chunks and slabs are its own."""
+    from graddft_amd import B3LYP_GRID, MLPSpec, NeuralFunctional
+    f = NeuralFunctional(MLPSpec(nc=6, h=32, n_hidden=2, nd=4))
+    a, b, c = _molecule(70, 9000, 1), _molecule(210, 90000, 2), _molecule(20, 700, 3)
+    for functional, theta in ((B3LYP_GRID, None), (f, f.init(1))):
+        for x, others in ((a, (b, c)), (c, (a, b)), (b, (a, c))):
+            print(f"case: the same in every batch, n={x.nao}, {precision}, kind {functional.kind}", flush=True)
+            alone = _batch_vxc([x], 0, precision, functional, theta)
+            beside = _batch_vxc([others[0], x, others[1]], 1, precision, functional, theta)
+            for u, v in zip(alone, beside):
+                assert torch.equal(u, v)
