@@ -33,9 +33,6 @@
 #include "gdx_rows.h"
 
 #include <algorithm>
-#include <map>
-#include <mutex>
-#include <tuple>
 #include <vector>
 
 namespace gdx {
@@ -613,12 +610,6 @@ __global__ __launch_bounds__(NT) void point_hvp_bwd_kernel(const double* __restr
 // ------------------------------------------------------------ workspace layout ----
 constexpr int NUM_CU = 256;    // MI355X compute units
 constexpr int RED_GROUPS = 32; // slice groups of the first reduction stage
-
-// V_xc output tile recorded by gdx_xc_autotune for a shape, keyed by (N_pad, n_pad, nsv, precision,
-// second order).  The build has one tile size, the best on every shape measured, so the record only
-// answers later calls.
-std::mutex vxc_tune_mu;
-std::map<std::tuple<int, int, int, int, int>, int> vxc_tune;
 
 // Tiling and chunks of one molecule in slabs of `slab` points, with about `budget` work items an XCD (spins counted): every class
 // of items starts with eight chunks, one an XCD, and the class whose items cost most gets eight more
@@ -1493,24 +1484,13 @@ int gdx_xc_forward(void* stream, const gdx_xc_desc* desc, const void* ao, const 
 }
 
 int gdx_xc_autotune(void* stream, const gdx_xc_desc* desc, const void* ao, void* workspace, int32_t* vt_inout) {
+  (void)stream;
   int rc = validate(desc);
   if (rc != GDX_OK) return rc;
   GDX_REQUIRE(ao && workspace, "gdx_xc_autotune: null pointer");
   const int pin = vt_inout ? *vt_inout : 0;
   GDX_REQUIRE(pin == 0 || pin == 64 || pin == 128, "gdx_xc_autotune: the tile may be pinned to 64 or 128 only");
-  if (pin != 0) {   // pinned by the caller: record without measuring
-    const bool nrl = is_neural(*desc);
-    const int nsv_fwd = (!nrl && desc->spin_restricted) ? 1 : 2;
-    std::lock_guard<std::mutex> g(vxc_tune_mu);
-    vxc_tune[std::make_tuple(desc->npts_pad, desc->nao_pad, nsv_fwd, desc->precision, 0)] = pin;
-    vxc_tune[std::make_tuple(desc->npts_pad, desc->nao_pad, 2, desc->precision, 1)] = pin;
-    return GDX_OK;
-  }
-  (void)stream;
-  const int nsv_fwd = (!is_neural(*desc) && desc->spin_restricted) ? 1 : 2;
-  std::lock_guard<std::mutex> g(vxc_tune_mu);
-  const auto known = vxc_tune.find(std::make_tuple(desc->npts_pad, desc->nao_pad, nsv_fwd, desc->precision, 0));
-  if (vt_inout) *vt_inout = known == vxc_tune.end() ? VX_CP : known->second;
+  if (vt_inout) *vt_inout = VX_CP;
   return GDX_OK;
 }
 

@@ -59,10 +59,6 @@ class MLPSpec:
         return 2 * sum(i * o for i, o in self.shapes())
 
 
-# Ask the library for the V_xc output tile of a plan's shape (gdx_xc_autotune) when it is created.
-AUTOTUNE = True
-
-
 def ao_planes_for(m: Molecule, precision: str) -> torch.Tensor:
     """AO planes in the element type of a precision: the FP64 planes, or their FP32 copy
     (made once and cached on the molecule), whose storage goes on with the bf16 plane of what
@@ -120,14 +116,6 @@ class XCPlan:
         self.generation = 0
         self.fwd_generation = -1
         self.hvp_workspace = None
-        # V_xc output tile of this shape
-        self.vxc_tile = None
-        if AUTOTUNE and molecule.ao_planes.is_cuda and not torch.cuda.is_current_stream_capturing():
-            vt = ctypes.c_int32(0)
-            st = torch.cuda.current_stream(molecule.ao_planes.device).cuda_stream
-            _lib.check(lib.gdx_xc_autotune(st, ctypes.byref(d), self._ao().data_ptr(), self.workspace.data_ptr(),
-                                           ctypes.byref(vt)), "gdx_xc_autotune")
-            self.vxc_tile = int(vt.value)
 
     @staticmethod
     def _ptr(t: Optional[torch.Tensor]) -> int:

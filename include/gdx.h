@@ -106,10 +106,9 @@ int gdx_xc_workspace_size(const gdx_xc_desc* desc, size_t* bytes);
 int gdx_xc_forward(void* stream, const gdx_xc_desc* desc, const void* ao, const double* weights,
                    const double* rdm1, const double* params, double* exc, void* workspace);
 
-/* V_xc tile of this descriptor's shape (no counterpart in the reference).  The V_xc build uses one
- * output tile, 64, which was fastest on every shape it was measured at, so nothing is timed: vt_inout
- * (may be NULL) holds 0 on entry to ask, 64 or 128 to record an answer for the shape (N_pad, n_pad,
- * spins, precision), which later calls in this process return; on exit the recorded tile, else 64. */
+/* Output tile of the V_xc build (no counterpart in the reference).  There is one, 64, which was fastest
+ * on every shape it was measured at: nothing is timed, launched or recorded.  vt_inout (may be NULL) holds
+ * the tile asked for, 64 or 128 or 0 for none; on exit the tile that the build uses, whatever was asked. */
 int gdx_xc_autotune(void* stream, const gdx_xc_desc* desc, const void* ao, void* workspace, int32_t* vt_inout);
 
 /* Custom coefficient functions (the reference's Functional(coefficients=..., ...) with a user
