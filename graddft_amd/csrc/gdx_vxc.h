@@ -30,7 +30,6 @@ namespace gdx {
 struct VxcMol {
   const void* ao;      // (5, npts_pad, nP) planes in the element type
   float* z;            // FP32: (nsv, slab, nP) Z of the current slab
-  float* u;            // FP32: (nsv, slab) u as a pair (high, low)
   double* part;        // partial sums, (slots, nsv, nP, nP): see vxc_reduce_kernel
   long row0;           // first row of this molecule in every spin plane of the potentials
   long out_off;        // first element of its (2, n, n) output
@@ -101,8 +100,8 @@ __device__ __forceinline__ VxcMol vxc_find(const VxcMol* __restrict__ mols, int 
   return u.m;
 }
 
-// FP32: Z of every point of a slab, column and spin, once instead of once per tile row, and u as FP32
-// pairs; four columns of a row a thread.  HBM-bound: reads the five planes once, writes nsv.
+// FP32: Z of every point of a slab, column and spin, once instead of once per tile row; four columns of a
+// row a thread.  HBM-bound: reads the five planes once, writes nsv.
 __global__ __launch_bounds__(256) inline void vxc_zform_kernel(const VxcMol* __restrict__ mols, int nmol,
                                                                const VxcMol one, const double* __restrict__ vpt,
                                                                size_t vpt_rows, int nsv, int slab) {
@@ -122,12 +121,6 @@ __global__ __launch_bounds__(256) inline void vxc_zform_kernel(const VxcMol* __r
     for (int e = 0; e < 4; ++e) o[e] = (float)(v0 * (double)p[e] + v1 * (double)x[e] + v2 * (double)y[e] +
                                               v3 * (double)z[e] + v4 * (double)l[e]);
     *(gptr_w<f4>)((gptr_w<float>)M.z + s * zplane + i) = o;
-    if (i % M.nP == 0) {
-      const float h = (float)v[5];
-      gptr_w<float> w = (gptr_w<float>)M.u + 2 * ((long)s * M.slab + r);
-      w[0] = h;
-      w[1] = (float)(v[5] - (double)h);
-    }
   }
 }
 
@@ -213,23 +206,26 @@ __device__ __forceinline__ unsigned vxc_sym_mask(const VxcQuad& Q, bool share) {
   return __builtin_amdgcn_readfirstlane(m & Q.mask);
 }
 
-__device__ __forceinline__ float readlane_f32(float x, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+__device__ __forceinline__ double readlane_f64(double x, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                          __builtin_amdgcn_readlane(__double2loint(x), lane));
 }
 
 // FP32: both operands split into three bf16 terms while staged (gdx_gemm_split.h), a stage is 32
 // points of one product.  A block's products are summed from zero in FP32 over VX_FL stages and then
 // added to FP64 accumulators: the integrand cancels strongly near the nuclei (large Laplacian terms),
 // and FP32 sums over hundreds of points degrade reverse mode through an SCF loop.  Staging takes as
-// many issue slots as the products (28% MFMA, 50% VALU busy at n = 560): row addresses stay scalar, u
-// is a pair of FP32 numbers held one point a lane and read by lane index.
+// many issue slots as the products (28% MFMA, 50% VALU busy at n = 560): row addresses stay scalar, u is
+// held one point a lane and read by lane index.  u d_j phi is an FP64 product rounded once (u as an FP32
+// pair: the same time, a second rounding, and no value past FP32's range).
 constexpr int VX_FL = 2;
 // Z is formed and multiplied a slab of points at a time, whose sums add to the partials of the slab
 // before (the same chunks of every slab, one launch after the other: a fixed order).  vxc_slabs has
 // the sizes.
 
 __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __restrict__ mols, int nmol,
-                                                                const VxcMol one, int nsv, int slab) {
+                                                                const VxcMol one, const double* __restrict__ vpt,
+                                                                size_t vpt_rows, int nsv, int slab) {
   __shared__ __align__(16) __bf16 Ls[3][4][VX_CP * 8];
   __shared__ __align__(16) __bf16 Rs[3][4][VX_CP * 8];
   const VxcMol M = vxc_find<&VxcMol::blk0>(mols, nmol, one, blockIdx.x);
@@ -246,12 +242,11 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
   // repeat the last one (their blocks are not computed)
   const unsigned cl = 4 * min(it.a0 * 16 + lane, nP - 1), cr = 4 * min(it.b0 * 16 + lane, nP - 1);
   const gptr<float> lp = (gptr<float>)M.ao;
-  const size_t r0 = (size_t)slab * M.slab;   // Z and u start with the slab
   const gptr<float> rp = sym ? lp : (gptr<float>)M.z + (size_t)it.s * M.slab * nP;
-  const size_t rs = sym ? 0 : r0 * nP;
-  const gptr<f2v> up = (gptr<f2v>)M.u + (size_t)it.s * M.slab + (lane & 31);
+  const size_t rs = sym ? 0 : (size_t)slab * M.slab * nP;   // Z starts with the slab
+  const gptr<double> up = (gptr<double>)vpt + ((size_t)it.s * vpt_rows + M.row0 + (lane & 31)) * VPT_STRIDE + 5;
   float xl[8], xr[8];
-  f2v u = {0.f, 0.f};   // u of point lane % 32 of the loaded stage
+  double u = 0.0;   // u of point lane % 32 of the loaded stage
   auto gload = [&](int pt, int pl) {
     const size_t row = pl * plane + (size_t)(pt + 8 * wave) * nP;
 #pragma unroll
@@ -259,7 +254,7 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
       xl[e] = row_load<float>(lp + row + e * nP, cl);
       xr[e] = row_load<float>(rp + (row - rs) + e * nP, cr);
     }
-    if (sym) u = up[pt - r0];
+    if (sym) u = up[(size_t)pt * VPT_STRIDE];
   };
   auto lstore = [&]() {
     bf8 f[3];
@@ -269,7 +264,7 @@ __global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __
     if (sym)
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        xr[e] = fmaf(readlane_f32(u[1], 8 * wave + e), xr[e], readlane_f32(u[0], 8 * wave + e) * xr[e]);
+        xr[e] = (float)(readlane_f64(u, 8 * wave + e) * (double)xr[e]);
     split8(xr, f[0], f[1], f[2]);
 #pragma unroll
     for (int p = 0; p < 3; ++p) *(bf8*)&Rs[p][wave][lane * 8] = f[p];

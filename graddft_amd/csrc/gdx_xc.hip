@@ -651,8 +651,8 @@ VxcMol vxc_plan(int Np, int nP, int nsv, int slab, double budget) {
 }
 // resident blocks an XCD: four a CU (FP32), two (FP64)
 inline int vxc_slots(bool fp64) { return NUM_CU / 8 * (fp64 ? 2 : 4); }
-// FP32 scratch: Z of `el` AO elements and u pairs of `rows` points a spin
-inline size_t vxc_z_bytes(size_t el, size_t rows, int nsv) { return nsv * (el * 4 + rows * 8); }
+// FP32 scratch: Z of a slab
+inline size_t vxc_z_bytes(int slab, int nP, int nsv) { return (size_t)nsv * slab * nP * 4; }
 // FP32: slabs of points, so that their Z takes no more than the MLP deltas over which it lies, or than
 // ZCAP (zbytes gives the scratch for a number of slabs).  Z of the whole grid was 2.0 GB at n = 560, 427k
 // points; V_xc of both spins takes 13.3 ms there with it, 11.8 in slabs of 128 MB (they stay in the
@@ -707,10 +707,7 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   L.rows = (int)R;
   const int nsv_max = hvp || neural || !d.spin_restricted ? 2 : 1;   // spins of V_xc builds
   L.Gbytes = neural ? 2 * R * d.mlp_h * es : 0;
-  auto zbytes = [&](int nslab) {
-    const size_t slab = vxc_slab((int)Np, nslab);
-    return vxc_z_bytes(slab * nP, slab, nsv_max);
-  };
+  auto zbytes = [&](int nslab) { return vxc_z_bytes(vxc_slab((int)Np, nslab), (int)nP, nsv_max); };
   L.nslab = batch || es == 8 ? 1 : vxc_slabs(zbytes, L.Gbytes);
   L.nchunk = 0;   // V_xc partial slots (chunks x nsv)
   for (int nsv = 1; nsv <= nsv_max; ++nsv)
@@ -764,8 +761,8 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   L.DX = take(neural ? R * d.mlp_nc * es : 0);
   L.vpt = take(2 * Np * VPT_STRIDE * 8);
   L.vpart = take(batch ? 0 : (size_t)L.nchunk * nP * nP * 8);
-  // FP32: Z, then the pairs of u, of a slab, over the MLP deltas where they are large enough (the V_xc
-  // build comes after the last use of G)
+  // FP32: Z of a slab, over the MLP deltas where they are large enough (the V_xc build comes after the
+  // last use of G)
   const size_t zslab = batch || es == 8 ? 0 : zbytes(L.nslab);
   L.Z = zslab <= L.Gbytes ? L.G : take(zslab);
   size_t wbytes = 0;
@@ -1033,7 +1030,7 @@ void launch_vxc_group(const Ctx& c, const VxcMol* mols, const VxcMol& one, const
   if constexpr (sizeof(T) == 4) {
     for (int slab = 0; slab < G.nslab; ++slab) {
       GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(G.zblocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
-      GDX_LAUNCH(nm, vxc_f32_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, nsv, slab);
+      GDX_LAUNCH(nm, vxc_f32_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
     }
   } else {
     GDX_LAUNCH(nm, vxc_f64_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv);
@@ -1165,7 +1162,6 @@ void launch_vxc(const Ctx& c, const T* ao, int nsv, double* d_rdm1) {
   VxcMol M = vxc_single<T>(d.npts_pad, d.nao_pad, nsv, c.L.nslab);
   M.ao = ao;
   M.z = c.P<float>(c.L.Z);
-  M.u = M.z + (size_t)nsv * M.slab * d.nao_pad;
   M.part = c.P<double>(c.L.vpart);
   M.n = d.nao;
   BatchCtx::Group G;
@@ -1643,7 +1639,7 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
   std::vector<size_t> zbytes_of(nmol, 0);
   for (int m = 0; m < nmol && es == 4; ++m) {
     const int Np = mols[m].npts_pad, nP = mols[m].nao_pad;
-    auto zbytes = [&](int k) { return vxc_z_bytes((size_t)vxc_slab(Np, k) * nP, vxc_slab(Np, k), 2); };
+    auto zbytes = [&](int k) { return vxc_z_bytes(vxc_slab(Np, k), nP, 2); };
     nslab[m] = vxc_slabs(zbytes, is_neural(d) ? 2 * (size_t)Np * d.mlp_h * es : 0);
     zbytes_of[m] = zbytes(nslab[m]);
   }
@@ -1748,7 +1744,6 @@ int gdx_xc_batch_create(const gdx_xc_desc* desc, int32_t nmol, const gdx_xc_batc
     for (int k = 0; k < 2; ++k) {
       vmol[k][m].part = (double*)(T0 + o_vp) + vpart_off[m];
       vmol[k][m].z = (float*)(Z0 + z_off[m]);
-      vmol[k][m].u = vmol[k][m].z + 2 * (size_t)vmol[k][m].slab * vmol[k][m].nP;
     }
   }
   for (int k = 0; k < 2; ++k) {
