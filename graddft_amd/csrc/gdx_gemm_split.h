@@ -132,12 +132,16 @@ __global__ void pack_weights_kernel(const double* __restrict__ params, long npar
 //   EPI_BIAS_ELU    C = ELU(A W + bias)
 //   EPI_ELU_BWD     C = (A W) elu'(Y), Y = the ELU output
 //   EPI_STORE       C = A W
+// An infinity, or a number past bf16's largest (3.39e38), has no split: its terms add up to NaN.  Such a
+// result is formed again from the FP32 operands (W at stride wk along k and wf along the features): a
+// unit saturated by it, ELU(-inf) = -1 or a coefficient of 0 or 2, is a finite answer.
 constexpr int GS_ROWS = 64;
 
 template <int NB, int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_split_kernel(int M, int h, const float* __restrict__ A,
-                                                            const __bf16* __restrict__ Wp, float* __restrict__ C,
-                                                            const float* __restrict__ bias,
+                                                            const __bf16* __restrict__ Wp,
+                                                            const float* __restrict__ W, int wk, int wf,
+                                                            float* __restrict__ C, const float* __restrict__ bias,
                                                             const float* __restrict__ Y) {
   // fragments [k-group][row], rows xored by twice the k-group: four lanes of a row store to different
   // banks, and a wave's reads stay conflict-free
@@ -203,6 +207,28 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(int M, int h, const 
       cur ^= 1;
       lstore(cur);
       __syncthreads();
+    }
+    f4 any = (f4)0.f;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) any += acc[j][i];
+    const float nan = (any[0] + any[1]) + (any[2] + any[3]);
+    if (__any(nan != nan)) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (j >= njv || acc[j][i][q] == acc[j][i][q]) continue;
+            const float* a = A + (size_t)min(m0 + i * 16 + r, M - 1) * h;
+            const float* w = W + (size_t)((jb0 + j) * 16 + 4 * g + q) * wf;
+            float s = 0.f;
+#pragma unroll 1
+            for (int k = 0; k < h; ++k) s = fmaf(a[k], w[(size_t)k * wk], s);
+            acc[j][i][q] = s;
+          }
     }
     // epilogue: feature f .. f + 3 of row m0 + 16 i + r
 #pragma unroll

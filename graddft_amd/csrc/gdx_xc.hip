@@ -836,7 +836,7 @@ void launch_layer(hipStream_t st, const char* name, int M, int h, const T* A, co
     // persistent blocks: as many as the registers leave resident (three a CU up to 128 features)
     const dim3 grid(std::min((M + GS_ROWS - 1) / GS_ROWS, NUM_CU * (h <= 128 ? 3 : 2)));
 #define GDX_SPLIT(NB)                                                                                           \
-  GDX_LAUNCH(name, (gemm_split_kernel<NB, EPI>), grid, dim3(NT), 0, st, M, h, A, Wp, C, bias, Y)
+  GDX_LAUNCH(name, (gemm_split_kernel<NB, EPI>), grid, dim3(NT), 0, st, M, h, A, Wp, W, TB ? 1 : h, TB ? h : 1, C, bias, Y)
     if (h <= 64) GDX_SPLIT(1);
     else if (h <= 128) GDX_SPLIT(2);
     else if (h <= 192) GDX_SPLIT(3);

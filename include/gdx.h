@@ -30,9 +30,12 @@ enum {
 /* Element type of the matrix products (densities, V_xc, MLP layers).  Per-point functional
  * math, contractions and every reduction over grid points are FP64 in all modes.
  *  GDX_FP64   all products FP64 (v_mfma_f64_16x16x4f64)
- *  GDX_FP32   FP32 operands and sums, FP32 AO planes: v_mfma_f32_16x16x4f32 for the densities; for
- *             V_xc and the MLP's hidden h x h layers every FP32 operand split into three bf16 terms,
- *             six products on v_mfma_f32_16x16x32_bf16, FP32 sums (at least FP32's accuracy)
+ *  GDX_FP32   FP32 AO planes, activations and potentials' products; rho and its gradient from FP64
+ *             products of the widened planes and D (v_mfma_f64_16x16x4f64); the kinetic term, V_xc and the
+ *             MLP's hidden h x h layers with every FP32 operand split into three bf16 terms, six products
+ *             on v_mfma_f32_16x16x32_bf16, FP32 sums (V_xc: FP64 from every 64 k on).  Layer results keep
+ *             infinities; an infinite AO derivative, activation or delta gives NaN, not an infinity, in the
+ *             gradients and in the kinetic term.
  *  GDX_BF16X6 the same kernels as GDX_FP32. */
 enum { GDX_FP64 = 0, GDX_FP32 = 1, GDX_BF16X6 = 2 };
 /* Or-ed into GDX_FP32 or GDX_BF16X6: the buffer of the five float AO planes goes on with a plane
