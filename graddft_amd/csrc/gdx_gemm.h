@@ -44,8 +44,7 @@ __device__ __forceinline__ double elu_any(double x) { return elu_d(x); }
 __device__ __forceinline__ float elu_any(float x) { return elu_f(x); }
 
 constexpr int GT_M = 128, GT_N = 128;
-// k per pipeline stage (32 measured slower)
-template <typename T> struct GemmK { static constexpr int value = 16; };
+constexpr int GT_K = 16;   // k per pipeline stage (32 measured slower)
 
 // Tile b and K-split of this block, with blocks sharing operands placed on one XCD (the
 // hardware dispatches linear block L to XCD L % 8, and each XCD has its own L2):
@@ -77,28 +76,26 @@ __device__ __forceinline__ void split_range(int y, int kchunk, int kseg, int sps
   if (kend < kbeg) kend = kbeg;
 }
 
-// Two blocks per CU: the 128 x 128 FP64 accumulators then live in VGPRs (256, no spills; 75-82 KB LDS a block), 28% faster for the
-// forward GEMM than one block with AGPR accumulators.
-template <typename T, bool TA, bool TB, int EPI>
+// Two blocks per CU: the 128 x 128 FP64 accumulators then live in VGPRs (256, no spills; 75-82 KB LDS a
+// block), 28% faster for the forward GEMM than one block with AGPR accumulators.
+template <bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
-    int M, int N, const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb,
-    T* __restrict__ C, int ldc, const T* __restrict__ bias, const T* __restrict__ Y, int ldy,
-    int kchunk, T* __restrict__ colsum, int kseg, int sps, const T* __restrict__ X16 = nullptr,
+    int M, int N, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb,
+    double* __restrict__ C, int ldc, const double* __restrict__ bias, const double* __restrict__ Y, int ldy,
+    int kchunk, double* __restrict__ colsum, int kseg, int sps, const double* __restrict__ X16 = nullptr,
     double* __restrict__ w0part = nullptr, int ncp = 0) {
-  typedef typename MfmaT<T>::acc_t acc_t;
-  constexpr int GT_K = GemmK<T>::value;
-  constexpr int VEC = 16 / sizeof(T);                // elements per 16-byte load
+  typedef MfmaT<double> Mfma;
+  constexpr int VEC = 2;                             // elements per 16-byte load
   constexpr int NVA = GT_M * GT_K / VEC / 256;       // vector loads per thread per tile
   constexpr int NVB = GT_N * GT_K / VEC / 256;
-  typedef T vec_t __attribute__((ext_vector_type(VEC)));
-  typedef T v4_t __attribute__((ext_vector_type(4)));
+  typedef double vec_t __attribute__((ext_vector_type(VEC)));
   // LDS tiles keep the global orientation (16-byte stores, no transposition):
   //   A: TA ? [k][m] (row GT_M + 4) : [m][k] (row GT_K + 4);  B: TB ? [n][k] : [k][n]
   constexpr int AKM = GT_M + 4, AMK = GT_K + 4, BKN = GT_N + 4, BNK = GT_K + 4;
   constexpr int ABUF = TA ? GT_K * AKM : GT_M * AMK;
   constexpr int BBUF = TB ? GT_N * BNK : GT_K * BKN;
-  __shared__ __align__(16) T As[2 * ABUF];
-  __shared__ __align__(16) T Bs[2 * BBUF];
+  __shared__ __align__(16) double As[2 * ABUF];
+  __shared__ __align__(16) double Bs[2 * BBUF];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
@@ -162,19 +159,19 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
   // in each 16-k half of the stage, k-group lane / 16 supplies k = 4 g + kk to MFMA step kk
   // (a permutation of those 16 k, the same for both operands), so a [m][k] or [n][k] tile is
   // read with one 4-element vector per fragment
-  auto afrag = [&](int buf, int m, int g, T* out) {
+  auto afrag = [&](int buf, int m, int g, double* out) {
     if (TA) {
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) out[kk] = As[buf * ABUF + (4 * g + kk) * AKM + m];
     } else {
-      const v4_t v = *(const v4_t*)&As[buf * ABUF + m * AMK + 4 * g];
+      const d4 v = *(const d4*)&As[buf * ABUF + m * AMK + 4 * g];
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) out[kk] = v[kk];
     }
   };
-  auto bfrag = [&](int buf, int n, int g, T* out) {
+  auto bfrag = [&](int buf, int n, int g, double* out) {
     if (TB) {
-      const v4_t v = *(const v4_t*)&Bs[buf * BBUF + n * BNK + 4 * g];
+      const d4 v = *(const d4*)&Bs[buf * BBUF + n * BNK + 4 * g];
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) out[kk] = v[kk];
     } else {
@@ -183,16 +180,16 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
     }
   };
 
-  acc_t acc[4][4];
+  d4 acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (acc_t){0, 0, 0, 0};
-  T csum = 0;
+    for (int j = 0; j < 4; ++j) acc[i][j] = (d4){0, 0, 0, 0};
+  double csum = 0;
   constexpr bool ELUB = EPI == EPI_ELU_BWD || EPI == EPI_ELU_BWD_W0, W0 = EPI == EPI_ELU_BWD_W0;
-  acc_t wacc[W0 ? 4 : 1];
+  d4 wacc[W0 ? 4 : 1];
 #pragma unroll
-  for (int j = 0; j < (W0 ? 4 : 1); ++j) wacc[j] = (acc_t){0, 0, 0, 0};
+  for (int j = 0; j < (W0 ? 4 : 1); ++j) wacc[j] = (d4){0, 0, 0, 0};
   if (nk > 0) {
     gload(kbeg);
     lstore(0);
@@ -208,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
 #pragma unroll
     for (int kb = 0; kb < GT_K / 16; ++kb) {
       const int g = kb * 4 + (lane >> 4), r = lane & 15;
-      T af[4][4], bf[4][4];
+      double af[4][4], bf[4][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) afrag(cur, wm + i * 16 + r, g, af[i]);
 #pragma unroll
@@ -218,14 +215,14 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = MfmaT<T>::op(af[i][kk], bf[j][kk], acc[i][j]);
+          for (int j = 0; j < 4; ++j) acc[i][j] = Mfma::op(af[i][kk], bf[j][kk], acc[i][j]);
     }
     if (kt + 1 < nk) lstore(cur ^ 1);
     __syncthreads();
   }
   if (colsum != nullptr && m0 == 0 && tid < GT_N) colsum[(size_t)ysplit * N + n0 + tid] = csum;
 
-  T* Cz = C + (size_t)ysplit * M * ldc;
+  double* Cz = C + (size_t)ysplit * M * ldc;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -233,17 +230,17 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
       const int col = n0 + wn + j * 16 + (lane & 15);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int row = m0 + wm + i * 16 + MfmaT<T>::row(lane, q);
-        T v = acc[i][j][q];
-        if (EPI == EPI_BIAS_ELU) v = elu_any(v + bias[col]);
+        const int row = m0 + wm + i * 16 + Mfma::row(lane, q);
+        double v = acc[i][j][q];
+        if (EPI == EPI_BIAS_ELU) v = elu_d(v + bias[col]);
         if constexpr (ELUB) {
-          const T y = Y[(size_t)row * ldy + col];
-          v *= (y > (T)0 ? (T)1 : y + (T)1);
+          const double y = Y[(size_t)row * ldy + col];
+          v *= (y > 0.0 ? 1.0 : y + 1.0);
         }
         if constexpr (W0) {
           // A = G^T (f = lane % 16, row slot lane / 16), B = X16 rows of the same slots
-          const T xr = X16[(size_t)row * 16 + (lane & 15)];
-          wacc[W0 ? j : 0] = MfmaT<T>::op(v, xr, wacc[W0 ? j : 0]);
+          const double xr = X16[(size_t)row * 16 + (lane & 15)];
+          wacc[W0 ? j : 0] = Mfma::op(v, xr, wacc[W0 ? j : 0]);
         }
         Cz[(size_t)row * ldc + col] = v;
       }
@@ -256,7 +253,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int f = n0 + wn + j * 16 + MfmaT<T>::row(lane, q);
+          const int f = n0 + wn + j * 16 + Mfma::row(lane, q);
           w0part[((size_t)slice * ncp + c) * N + f] = (double)wacc[W0 ? j : 0][q];
         }
     }

@@ -84,7 +84,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_narrow_kernel(int M, int h, c
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         v[q] = acc[j][q];
-        if (EPI == EPI_BIAS_ELU) v[q] = elu_any(v[q] + bias[n + q]);
+        if (EPI == EPI_BIAS_ELU) v[q] = elu_d(v[q] + bias[n + q]);
         if (EPI == EPI_ELU_BWD) {
           const double y = Y[row + n + q];
           v[q] *= y > 0.0 ? 1.0 : y + 1.0;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_narrow_kernel(int M, int h, c
 
 // part[z] (h x h) = H^T G over split z of the rows, colsum[z] the column sums of G; grid (ceil(h / 64),
 // ceil(h / 64), splits).  Splits are whole groups of 16 rows.
-__global__ __launch_bounds__(256, 2) inline void wgrad_narrow_kernel(int h, const double* __restrict__ H,
+__global__ __launch_bounds__(256, 2) void wgrad_narrow_kernel(int h, const double* __restrict__ H,
                                                                      const double* __restrict__ G,
                                                                      double* __restrict__ part,
                                                                      double* __restrict__ colsum, int kchunk, int kseg,

@@ -86,7 +86,7 @@ __device__ __forceinline__ void mfma_chain(const bf8 (&a)[3], const bf8 (&b)[3],
 __host__ __device__ inline int split_ksteps(int h) { return (h + 31) / 32; }
 inline size_t split_pack_elems(int h) { return (size_t)split_ksteps(h) * (h / 16) * 3 * 64 * 8; }
 
-// All parameters to FP32 (biases and edge layers read that copy), then for each hidden layer
+// All parameters to FP32 (the hidden biases and the rows formed again read that copy), then for each hidden layer
 // l = 1 .. nl-1 the packed W_l (forward: feature = output, k = input) and W_l^T (backward) at
 // pack + (2 (l - 1) + direction) * split_pack_elems(h).  w1 = offset of W_1, layer stride h h + h.
 __global__ void pack_weights_kernel(const double* __restrict__ params, long nparam, float* __restrict__ lowp,

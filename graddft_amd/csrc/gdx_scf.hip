@@ -65,18 +65,17 @@ __device__ __forceinline__ void coulomb_tile_of(long x, long& bi, long& bk) {
   bk = x - bi * (bi + 1) / 2;
 }
 
-template <int TT>
 __global__ __launch_bounds__(NT) void coulomb_tile_kernel(const double* __restrict__ eri, long P,
                                                           const double* __restrict__ Dt,
                                                           double* __restrict__ prow, double* __restrict__ pcol) {
-  // TT x TT tile of the lower triangle; 256 threads as 16 (ty) x 16 (tx); rows I = I0 + ty + 16 a,
+  // small (JTS) tile of the lower triangle; 256 threads as 16 (ty) x 16 (tx); rows I = I0 + ty + 16 a,
   // columns K = K0 + 16 j + tx
-  constexpr int NA = TT / 16;
-  __shared__ double cs[16][TT + 1];
+  constexpr int NA = JTS / 16;
+  __shared__ double cs[16][JTS + 1];
   long bi, bk;
   coulomb_tile_of(blockIdx.x, bi, bk);
   const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  const long I0 = bi * TT, K0 = bk * TT;
+  const long I0 = bi * JTS, K0 = bk * JTS;
   double dk[NA], csum[NA];
 #pragma unroll
   for (int j = 0; j < NA; ++j) {
@@ -85,7 +84,7 @@ __global__ __launch_bounds__(NT) void coulomb_tile_kernel(const double* __restri
     csum[j] = 0.0;
   }
   double rsum[NA];
-  if (bk < bi && I0 + TT <= P) {
+  if (bk < bi && I0 + JTS <= P) {
     // every K < every I of the tile, every I < P
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
@@ -134,7 +133,7 @@ __global__ __launch_bounds__(NT) void coulomb_tile_kernel(const double* __restri
 #pragma unroll
   for (int j = 0; j < NA; ++j) cs[ty][j * 16 + tx] = csum[j];
   __syncthreads();
-  for (int k = tid; k < TT; k += NT) {
+  for (int k = tid; k < JTS; k += NT) {
     const long K = K0 + k;
     double c = 0.0;
 #pragma unroll
@@ -534,11 +533,6 @@ __global__ __launch_bounds__(NXC_THREADS) void scf_status_kernel(int n, const do
     if (energy && !isfinite(*energy)) bits |= 2;
     if (bits) atomicOr(status, bits);
   }
-}
-
-__global__ void zero_kernel(double* __restrict__ p, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
 }
 
 // ------------------------------------------------------------- Cholesky ---------------
@@ -1347,7 +1341,7 @@ void packed_product(hipStream_t st, const char* name, const double* m, long P, c
   const long nb = (P + tt - 1) / tt;
   const dim3 grid((unsigned)(nb * (nb + 1) / 2 * R));
   if (tt == JTS)
-    GDX_LAUNCH(name, coulomb_tile_kernel<JTS>, grid, dim3(NT), 0, st, m, P, v, prow, pcol);
+    GDX_LAUNCH(name, coulomb_tile_kernel, grid, dim3(NT), 0, st, m, P, v, prow, pcol);
   else if (R == 1)
     GDX_LAUNCH(name, coulomb_rows_kernel<JT>, grid, dim3(NT), 0, st, m, P, v, prow, pcol);
   else

@@ -102,7 +102,7 @@ __device__ __forceinline__ VxcMol vxc_find(const VxcMol* __restrict__ mols, int 
 
 // FP32: Z of every point of a slab, column and spin, once instead of once per tile row; four columns of a
 // row a thread.  HBM-bound: reads the five planes once, writes nsv.
-__global__ __launch_bounds__(256) inline void vxc_zform_kernel(const VxcMol* __restrict__ mols, int nmol,
+__global__ __launch_bounds__(256) void vxc_zform_kernel(const VxcMol* __restrict__ mols, int nmol,
                                                                const VxcMol one, const double* __restrict__ vpt,
                                                                size_t vpt_rows, int nsv, int slab) {
   const VxcMol M = vxc_find<&VxcMol::zblk0>(mols, nmol, one, blockIdx.x);
@@ -223,7 +223,7 @@ constexpr int VX_FL = 2;
 // before (the same chunks of every slab, one launch after the other: a fixed order).  vxc_slabs has
 // the sizes.
 
-__global__ __launch_bounds__(256, 4) inline void vxc_f32_kernel(const VxcMol* __restrict__ mols, int nmol,
+__global__ __launch_bounds__(256, 4) void vxc_f32_kernel(const VxcMol* __restrict__ mols, int nmol,
                                                                 const VxcMol one, const double* __restrict__ vpt,
                                                                 size_t vpt_rows, int nsv, int slab) {
   __shared__ __align__(16) __bf16 Ls[3][4][VX_CP * 8];
@@ -462,7 +462,7 @@ __device__ __forceinline__ void vxc_f64_item(const VxcMol& M, const VxcItem& it,
       }
 }
 
-__global__ __launch_bounds__(256, 2) inline void vxc_f64_kernel(const VxcMol* __restrict__ mols, int nmol,
+__global__ __launch_bounds__(256, 2) void vxc_f64_kernel(const VxcMol* __restrict__ mols, int nmol,
                                                                 const VxcMol one, const double* __restrict__ vpt,
                                                                 size_t vpt_rows, int nsv) {
   __shared__ __align__(16) double Is[5][VXD_K][VXD_LD];   // tile I: phi, its derivatives, Z

@@ -11,15 +11,16 @@
 //                    per-point product and of the weights; FP64 sum)
 //   dE/dD            train.py:86-121 (value_and_grad w.r.t. rdm1, unsymmetrised)
 //
-// Precision: the matrix products (density X = A D, V_xc, MLP layers) run on MFMA in the
-// element type T of the path -- double (GDX_FP64) or float (GDX_FP32); the per-point
-// functional math, the density row contractions, every reduction over grid points or
-// split partials and the E_xc sum are FP64 in both paths.
+// Precision: T is the element type of AO planes and activations, double (GDX_FP64) or float.  Matrix
+// products run on MFMA, in FP64 for double; for float the densities' X = phi D too, and V_xc, the
+// kinetic term and the MLP layers on three-term bf16 splits with FP32 sums.  The per-point functional
+// math, the density row contractions, every reduction over grid points or split partials and the E_xc
+// sum are FP64 in both paths.
 //
-// Kernel sequence, forward:  pad_dm -> density -> point_fwd -> [layer0 -> gemm_tile
+// Kernel sequence, forward:  dens_pack -> density -> point_fwd -> [layer0 -> layer
 //   (bias+ELU) x (L-1) -> head_fwd (skinny MFMA + coefficient/energy epilogue)] -> reduce.
 // Backward:  head_seed -> [head_delta -> skinny_wgrad (last layer) -> per hidden layer
-//   gemm_tile wgrad (split-K) + gemm_tile bwd-data (ELU') -> layer0_bwd (skinny) +
+//   wgrad (split-K) + bwd-data (ELU') -> layer0_bwd (skinny) +
 //   skinny_wgrad (first layer)] -> point_bwd (duals) -> vxc -> reduce_vxc.
 #include "gdx_common.h"
 #include "gdx_functionals.h"
@@ -66,7 +67,6 @@ inline LinCoef lin_coef(const gdx_xc_desc& d) {
 }
 
 __device__ __forceinline__ double clip30(double x) { return fabs(x) > 1e-30 ? x : 0.0; }
-__device__ __forceinline__ double elu_grad_from_out(double y) { return y > 0.0 ? 1.0 : y + 1.0; }
 
 __device__ __forceinline__ double block_sum(double v, double* red) {
   v = warp_sum(v);
@@ -702,7 +702,6 @@ Layout make_layout(const gdx_xc_desc& d, bool hvp = false, bool batch = false) {
   const size_t R = hvp ? 2 * Np : Np;  // rows of the activation-side buffers
   const size_t es = elem_size(d.precision);
   const bool neural = is_neural(d);
-  const int hmode = d.kind == GDX_FUNC_B3LYP_NEURAL_CORR ? 1 : 0;
   L.nsd = d.spin_restricted ? 1 : 2;
   L.rows = (int)R;
   const int nsv_max = hvp || neural || !d.spin_restricted ? 2 : 1;   // spins of V_xc builds
@@ -832,7 +831,8 @@ const char* gname(const gdx_xc_desc& d, const char* f64, const char* f32, const 
 template <typename T, bool TB, int EPI>
 void launch_layer(hipStream_t st, const char* name, int M, int h, const T* A, const T* W, const __bf16* Wp, T* C,
                   const T* bias, const T* Y, const T* X16 = nullptr, double* w0part = nullptr, int ncp = 0) {
-  if constexpr (sizeof(T) == 4 && EPI != EPI_ELU_BWD_W0) {
+  static_assert(sizeof(T) == 8 || EPI != EPI_ELU_BWD_W0, "the fused first-layer gradient is FP64's");
+  if constexpr (sizeof(T) == 4) {
     // persistent blocks: as many as the registers leave resident (three a CU up to 128 features)
     const dim3 grid(std::min((M + GS_ROWS - 1) / GS_ROWS, NUM_CU * (h <= 128 ? 3 : 2)));
 #define GDX_SPLIT(NB)                                                                                           \
@@ -842,11 +842,10 @@ void launch_layer(hipStream_t st, const char* name, int M, int h, const T* A, co
     else if (h <= 192) GDX_SPLIT(3);
     else GDX_SPLIT(4);
 #undef GDX_SPLIT
-  } else if constexpr (sizeof(T) == 4) {
   } else if (M % GT_M == 0 && h % GT_N == 0) {   // (h = 128, 73k rows: 78-86 us a layer, narrow kernel 92)
     const dim3 grid((M / GT_M) * (h / GT_N), 1);
-    GDX_LAUNCH(name, (gemm_tile_kernel<T, false, TB, EPI>), grid, dim3(NT), 0, st, M, h, A, h, W, h, C, h, bias, Y, h,
-               h, (T*)nullptr, h, 1, X16, w0part, ncp);
+    GDX_LAUNCH(name, (gemm_tile_kernel<false, TB, EPI>), grid, dim3(NT), 0, st, M, h, A, h, W, h, C, h, bias, Y, h,
+               h, (double*)nullptr, h, 1, X16, w0part, ncp);
   } else {
     if constexpr (EPI != EPI_ELU_BWD_W0) {
       // persistent blocks, as many as the weights in LDS leave resident (four, two and one a CU)
@@ -876,8 +875,8 @@ void launch_wgrad(hipStream_t st, const char* name, int rows, int h, const Layou
   } else if (h > 128 && h % GT_N == 0) {   // (h = 256, 73k rows: 170 us, narrow kernel 182 at h = 240;
                                            // h = 128: 95, narrow kernel 54)
     const dim3 grid((h / GT_M) * (h / GT_N), L.nsplit);
-    GDX_LAUNCH(name, (gemm_tile_kernel<T, true, false, EPI_STORE>), grid, dim3(NT), 0, st, h, h, Hin, h, G, h, part, h,
-               (const T*)nullptr, (const T*)nullptr, 0, L.kchunk, colsum, L.kseg, L.sps);
+    GDX_LAUNCH(name, (gemm_tile_kernel<true, false, EPI_STORE>), grid, dim3(NT), 0, st, h, h, Hin, h, G, h, part, h,
+               (const double*)nullptr, (const double*)nullptr, 0, L.kchunk, colsum, L.kseg, L.sps);
   } else {
     const dim3 grid((h + 63) / 64, (h + 63) / 64, L.nsplit);
     GDX_LAUNCH("wgrad_narrow", wgrad_narrow_kernel, grid, dim3(NT), 0, st, h, Hin, G, part, colsum, L.kchunk, L.kseg,
@@ -907,7 +906,7 @@ ParamOffsets param_offsets(const gdx_xc_desc& d) {
 // A batch of molecules (one functional, one precision, different grids and bases) runs as one
 // evaluation: every per-point buffer is the concatenation of the molecules' rows (each
 // molecule's npts_pad a multiple of 256, so every 256-, 128- and 64-row block belongs to one
-// molecule), the MLP GEMMs run once over all rows, and the AO-side kernels (padding of D, the
+// molecule), the MLP GEMMs run once over all rows, and the AO-side kernels (packing of D, the
 // density kernel, V_xc and its reduction) are single launches over a ragged queue of
 // (molecule, tile) work items.  Per-molecule scalars (E_xc, edot) are segment sums of the
 // block partials; per-molecule cotangents enter as per-point scales.
@@ -1007,7 +1006,7 @@ void launch_density(const Ctx& c, const T* ao, const double* mats, bool tangent,
     blocks = dens_blocks(d.npts_pad, nspin);
     pblocks = (int)((dens_pack_threads<T>(d.nao_pad, nspin) + 255) / 256);
   }
-  GDX_LAUNCH("pad_dm", dens_pack_kernel<T>, dim3(pblocks), dim3(256), 0, st, mols, nmol, one, nspin, mats);
+  GDX_LAUNCH("dens_pack", dens_pack_kernel<T>, dim3(pblocks), dim3(256), 0, st, mols, nmol, one, nspin, mats);
   const char* nm = tname<T>("density_f64", "density_f32");
   if constexpr (sizeof(T) == 4) {
     if (d.precision & GDX_AO_LOW) {
@@ -1049,9 +1048,8 @@ void launch_vxc_batch(const Ctx& c, int nsv, double* d_rdm1) {
 template <typename T>
 void run_densities(const Ctx& c, const T* ao, const double* rdm1, const double* weights, double* dens_fin) {
   const gdx_xc_desc& d = c.d;
-  const int Np = d.npts_pad, nP = d.nao_pad;
+  const int Np = d.npts_pad;
   const bool neural = is_neural(d);
-  const int hmode = d.kind == GDX_FUNC_B3LYP_NEURAL_CORR ? 1 : 0;
   hipStream_t st = c.st;
   launch_density<T>(c, ao, rdm1, false, c.L.nsd, c.P<double>(c.L.dens_part));
   GDX_LAUNCH("point_fwd", point_fwd_kernel<T>, dim3(c.L.npt_blocks), dim3(NT), 0, st, c.P<double>(c.L.dens_part),
@@ -1237,7 +1235,7 @@ int backward_impl(const Ctx& c, const T* ao, const double* weights, const double
   hipStream_t st = c.st;
   const bool neural = is_neural(d);
   const int hmode = d.kind == GDX_FUNC_B3LYP_NEURAL_CORR ? 1 : 0;
-  const int Np = d.npts_pad, nP = d.nao_pad;
+  const int Np = d.npts_pad;
   const int nd = 4;
   if (neural) {
     const int h = d.mlp_h;
@@ -1292,11 +1290,14 @@ int backward_impl(const Ctx& c, const T* ao, const double* weights, const double
       // delta for layer l's input: (Gcur W_l^T) * elu'(Hin); for l = 1 that delta's first-layer
       // weight-gradient partials come out of the same epilogue (w0_fused)
       const __bf16* Wp = packed_weights<T>(c, l, true);
-      if (l == 1 && w0_fused)
-        launch_layer<T, true, EPI_ELU_BWD_W0>(
-            st, "gemm_f64_bwd_data_w0", Np, h, Gcur, Wl, Wp,
-            Gnext, nullptr, Hin, c.P<T>(L.X), c.P<double>(L.wpart), d.mlp_nc + 1);
-      else
+      bool fused = false;
+      if constexpr (sizeof(T) == 8) {
+        fused = l == 1 && w0_fused;
+        if (fused)
+          launch_layer<T, true, EPI_ELU_BWD_W0>(st, "gemm_f64_bwd_data_w0", Np, h, Gcur, Wl, Wp, Gnext, nullptr, Hin,
+                                                c.P<T>(L.X), c.P<double>(L.wpart), d.mlp_nc + 1);
+      }
+      if (!fused)
         launch_layer<T, true, EPI_ELU_BWD>(st, gname<T>(d, "gemm_f64_bwd_data", "gemm_f32_bwd_data", "gemm_bf16x6_bwd_data"),
                                            Np, h, Gcur, Wl, Wp, Gnext, nullptr, Hin);
       std::swap(Gcur, Gnext);
@@ -1349,7 +1350,7 @@ int hvp_impl(const Ctx& c, const T* ao, const double* weights, const double* rdm
   hipStream_t st = c.st;
   const bool neural = is_neural(d);
   const int hmode = d.kind == GDX_FUNC_B3LYP_NEURAL_CORR ? 1 : 0;
-  const int Np = d.npts_pad, nP = d.nao_pad;
+  const int Np = d.npts_pad;
   const int nd = 4;
   double* scal = c.b ? c.b->scal : c.P<double>(L.scal);
   int rc = forward_impl<T>(c, ao, weights, rdm1, params, exc ? exc : scal);
