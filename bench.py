@@ -27,21 +27,44 @@ import time
 import numpy as np
 
 METRIC = "XC grid pts/s (fwd+adjoint) & ms/SCF iter at ≤1e-6 Ha vs FP64 GPU path"
-PEAK = {"fp64": ("TFLOP/s", 78.6), "fp32": ("TFLOP/s", 157.3), "bf16x6": ("TFLOP/s", 2500.0)}
+# dense MFMA peaks, TFLOP/s, and the unit of a precision's dominant products
+PEAK = {"f64": 78.6, "f32": 157.3, "bf16": 2500.0}
 DTYPE = {"fp64": "f64", "fp32": "f32", "bf16x6": "bf16x6"}
 
 
+def grid_work(npts, n, nsd, nsv, f_mlp, precision):
+    """Matrix products of densities of nsd spins, V_xc of nsv spins and f_mlp network flops a point, as
+    {unit: flops that the unit executes}.  The terms in the AO derivatives are symmetric forms: with
+    phi D (or phi^T Z) 2 n^2 and half of the derivatives' 6 n^2, 5 n^2 a spin each way.  FP64 runs all of it
+    on the FP64 MFMA; FP32 and BF16X6 phi D there, everything else as six bf16 products each."""
+    if precision == "fp64":
+        return {"f64": npts * (5 * n * n * (nsd + nsv) + f_mlp)}
+    return {"f64": npts * 2 * n * n * nsd, "bf16": 6 * npts * (3 * n * n * nsd + 5 * n * n * nsv + f_mlp)}
+
+
+def floor_s(work):
+    """Time of the executed flops at their units' peaks, one unit after the other."""
+    return sum(f / (PEAK[u] * 1e12) for u, f in work.items())
+
+
+def against_floor(work, seconds):
+    """Executed rate against the peak of that mix of units; frac = floor / measured."""
+    flops, t = sum(work.values()), floor_s(work)
+    return {"achieved": round(flops / seconds / 1e12, 3), "peak": round(flops / t / 1e12, 1), "unit": "TFLOP/s",
+            "frac": round(t / seconds, 4), "floor_us": round(t * 1e6, 2),
+            "executed_flops": {u: int(f) for u, f in work.items()}}
+
+
 def scf_roofline(npts, n, nsd, f_mlp, ms_per_iter, precision):
-    """ms per SCF iteration against the roofline: algorithmic work per iteration W = N (n_s 16 n^2
-    + 2 F_mlp) flops (density phi D and grad-phi D, V_xc, the MLP forward and its adjoint) at
-    the precision's peak (FP64 78.6 TF/s; FP32 MFMA 157.3 TF/s for fp32 and bf16x6, whose grid
-    GEMMs run in FP32), plus the packed ERI read once (8 n_pack bytes) at 8 TB/s."""
+    """ms per SCF iteration against the roofline: the grid's matrix products (densities, V_xc, the network
+    forward and its adjoint, grid_work) at their units' peaks, plus the packed ERI read once (8 n_pack
+    bytes) at 8 TB/s."""
     P = n * (n + 1) // 2
     eri_bytes = 8 * (P * (P + 1) // 2)
-    flops = npts * (nsd * 16 * n * n + 2 * f_mlp)
-    peak = 78.6e12 if precision == "fp64" else 157.3e12
-    t_c, t_m = flops / peak, eri_bytes / 8e12
-    return {"flops_per_iter": int(flops), "eri_bytes_per_iter": int(eri_bytes), "peak_tflops": peak / 1e12,
+    work = grid_work(npts, n, nsd, nsd, 2 * f_mlp, precision)
+    t_c, t_m = floor_s(work), eri_bytes / 8e12
+    return {"executed_flops_per_iter": {u: int(f) for u, f in work.items()}, "eri_bytes_per_iter": int(eri_bytes),
+            "peaks_tflops": {u: PEAK[u] for u in work},
             "roofline_us": round((t_c + t_m) * 1e6, 2), "compute_us": round(t_c * 1e6, 2),
             "hbm_us": round(t_m * 1e6, 2), "measured_us": round(ms_per_iter * 1e3, 2),
             "frac": round((t_c + t_m) / (ms_per_iter / 1e3), 4)}
@@ -77,21 +100,23 @@ def parse():
     return ap.parse_args()
 
 
-def kernel_flops(name, npts, nao, spec, nsd):
-    """Algorithmic flops of ONE launch of the named kernel (N real points)."""
-    h = spec.h
-    table = {
-        "density": nsd * 8 * nao * nao * npts,       # 4 products (phi, dphi) x D
-        "vxc": 2 * 8 * nao * nao * npts,             # phi^T Z + 3 dphi^T u dphi, per spin
-        "gemm_fwd": 2 * npts * h * h,
-        "gemm_bwd_data": 2 * npts * h * h,
+def kernel_work(name, npts, nao, spec, nsd, precision):
+    """{unit: executed flops} of ONE launch of the named kernel (N real points), or None."""
+    layer = 2 * npts * spec.h * spec.h
+    flops = {
+        "gemm_fwd": layer, "gemm_bwd_data": layer, "gemm_wgrad": layer,
         # the last one also forms the first-layer weight gradient (7 columns incl. the bias)
-        "gemm_bwd_data_w0": 2 * npts * h * h + 2 * npts * h * (spec.nc + 1),
-        "gemm_wgrad": 2 * npts * h * h,
+        "gemm_bwd_data_w0": layer + 2 * npts * spec.h * (spec.nc + 1),
     }
     for suffix in ("_f64", "_f32", "_bf16x6"):
         name = name.replace(suffix, "")
-    return table.get(name)
+    if name == "density":
+        return grid_work(npts, nao, nsd, 0, 0, precision)
+    if name == "vxc":
+        return {u: f for u, f in grid_work(npts, nao, 0, 2, 0, precision).items() if f}
+    if name in flops:
+        return {"f64": flops[name]} if precision == "fp64" else {"bf16": 6 * flops[name]}
+    return None
 
 
 def cpu_baseline(mol, theta, spec, sample):
@@ -430,7 +455,7 @@ def config5_bench(args):
     theta = f.init(seed=6)
     N, n = mol.grid_size, mol.nao
     nsd = 1 if mol.restricted else 2
-    w_pt = 8 * n * n * nsd + 8 * n * n * 2 + 3 * spec.flops_per_point()
+    w_pt = 5 * n * n * nsd + 5 * n * n * 2 + 3 * spec.flops_per_point()
     out = {"workload": f"40 C (seeded, 12 A cube) def2-SVP nao={n}, grid level {level} ({N} pts), D from 120 "
                        "orbitals, MLP 3x256: E_xc + dE/dD + dE/dtheta", "npts": N, "nao": n, "inputs": inputs,
            "flop_per_point": w_pt}
@@ -452,13 +477,11 @@ def config5_bench(args):
             plan.backward(D, theta, one, dD, dth, plan.generation)
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t0) / reps * 1e3
-        # split-BF16 mixes bf16 products (hidden layers) with FP32 ones: no single peak
-        peak = PEAK[prec][1] if prec != "bf16x6" else None
         tf = w_pt * N / (ms / 1e3) / 1e12
         res[prec] = (float(exc), dD.clone(), dth.clone())
         out[prec] = {"ms_per_step": round(ms, 3), "grid_pts_per_s": round(N / (ms / 1e3), 1),
-                     "algorithmic_tflops": round(tf, 2), "peak": peak,
-                     "frac": round(tf / peak, 4) if peak else None}
+                     "algorithmic_tflops": round(tf, 2),
+                     **against_floor(grid_work(N, n, nsd, 2, 3 * spec.flops_per_point(), prec), ms / 1e3)}
         del plan
     e64, d64, t64 = res["fp64"]
     rel = lambda a, b: float(torch.linalg.norm(a - b) / torch.linalg.norm(b))  # noqa: E731
@@ -828,19 +851,15 @@ def main():
     # dominant kernel and its roofline
     name, (tot_ms, cnt) = max(kt.result.items(), key=lambda kv: kv[1][0])
     nsd = 1 if mol.restricted else 2
-    flops = kernel_flops(name, N, n, spec, nsd)
-    unit, peak = PEAK[args.precision]
+    work = kernel_work(name, N, n, spec, nsd, args.precision)
     roof = None
-    if flops is not None:
+    if work is not None:
         avg_s = tot_ms / cnt / 1e3
-        achieved = flops / avg_s / 1e12
         tr = measured_traffic().get(name)
-        roof = {"bound": "mfma", "kernel": name, "achieved": round(achieved, 3), "peak": peak,
-                "unit": unit, "frac": round(achieved / peak, 4), "traffic": tr,
+        roof = {"bound": "mfma", "kernel": name, **against_floor(work, avg_s), "traffic": tr,
                 "traffic_unit": "bytes per launch (HBM, rocprofv3 FETCH_SIZE/WRITE_SIZE scaled by a "
                                 "copy-kernel calibration; profiles/traffic_*.txt)" if tr else None,
-                "avg_launch_us": round(avg_s * 1e6, 2), "launches_per_step": cnt // args.steps,
-                "flops_per_launch": flops}
+                "avg_launch_us": round(avg_s * 1e6, 2), "launches_per_step": cnt // args.steps}
     # accuracy and speed against the plain FP64 GPU path on the same inputs
     vs64 = None
     if args.precision != "fp64":
@@ -894,8 +913,9 @@ def main():
             streaming[k] = {"bytes_per_launch": b, "avg_launch_us": round(tot / cnt * 1e3, 2),
                             "GB/s": round(gbs, 1), "frac_of_8TB/s": round(gbs / 8000.0, 3)}
     nsv = 2
-    w_pt = 8 * n * n * nsd + 8 * n * n * nsv + 3 * spec.flops_per_point()
+    w_pt = 5 * n * n * nsd + 5 * n * n * nsv + 3 * spec.flops_per_point()
     step_tflops = w_pt * N / (ms / 1e3) / 1e12
+    step_work = grid_work(N, n, nsd, nsv, 3 * spec.flops_per_point(), args.precision)
 
     def section(run, skip):
         # each section's molecules hold device memory until the cyclic collector frees them
@@ -948,8 +968,8 @@ def main():
         },
         "roofline": roof,
         "streaming": streaming,
-        "step_mfma": {"algorithmic_tflops": round(step_tflops, 3), "peak": peak,
-                      "frac": round(step_tflops / peak, 4), "flop_per_point": w_pt},
+        "step_mfma": {"algorithmic_tflops": round(step_tflops, 3), "flop_per_point": w_pt,
+                      **against_floor(step_work, ms / 1e3)},
         "kernels_ms_per_step": {k: round(v[0] / args.steps, 4) for k, v in
                                 sorted(kt.result.items(), key=lambda kv: -kv[1][0])},
         "vs_fp64_gpu": vs64,
