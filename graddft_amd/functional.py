@@ -72,8 +72,13 @@ def ao_planes_for(m: Molecule, precision: str) -> torch.Tensor:
         n = p[0].numel()   # even: the padded rows are a multiple of 64
         buf = torch.empty(5 * n + n // 2, dtype=torch.float32, device=p.device)
         a = buf[:5 * n].view(p.shape)
-        a.copy_(p)
-        torch.sub(p[0], a[0], out=buf[5 * n:].view(torch.bfloat16).view(p.shape[1:]))
+        if p.is_cuda and p.is_contiguous() and p.dtype == torch.float64 and p.data_ptr() % 32 == 0:
+            st = torch.cuda.current_stream(p.device).cuda_stream
+            _lib.check(_lib.load().gdx_ao_planes_f32(st, p.shape[1], p.shape[2], p.data_ptr(), buf.data_ptr()),
+                       "gdx_ao_planes_f32")
+        else:
+            a.copy_(p)
+            torch.sub(p[0], a[0], out=buf[5 * n:].view(torch.bfloat16).view(p.shape[1:]))
         m.cache[key] = a
     return a
 

@@ -94,6 +94,10 @@ int gdx_ao_eval(void* stream, int32_t nshell, const int32_t* shell_i32, const do
                 const double* prim_f64, const double* tmat_f64, int32_t npts, int32_t npts_pad,
                 const double* coords, int32_t nao, int32_t nao_pad, double* ao);
 
+/* The planes of GDX_FP32 and GDX_BF16X6 with GDX_AO_LOW from gdx_ao_eval's: ao_f32 takes 22 npts_pad nao_pad
+ * bytes (five float planes, then phi - (float)phi in bf16).  ao 32-byte, ao_f32 16-byte aligned. */
+int gdx_ao_planes_f32(void* stream, int32_t npts_pad, int32_t nao_pad, const double* ao, void* ao_f32);
+
 /* Bytes of device workspace gdx_xc_forward / gdx_xc_backward need for `desc`. */
 int gdx_xc_workspace_size(const gdx_xc_desc* desc, size_t* bytes);
 

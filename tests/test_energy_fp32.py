@@ -28,6 +28,20 @@ def test_fp32_planes_carry_the_remainder_of_phi():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(64, 16), (192, 48), (4160, 112)])
+def test_device_planes_are_the_host_s(rows, cols):
+    from types import SimpleNamespace
+    from graddft_amd.functional import ao_planes_for
+    planes = torch.randn(5, rows, cols, dtype=torch.float64) * 10.0 ** torch.randint(-30, 10, (5, rows, cols))
+    got = {}
+    for dev, p in (("cpu", planes), ("cuda", planes.cuda()), ("strided", planes.cuda().transpose(1, 2).contiguous().transpose(1, 2))):
+        a = ao_planes_for(SimpleNamespace(ao_planes=p, cache={}), "fp32")
+        got[dev] = torch.empty(0, dtype=torch.float32, device=a.device).set_(a.untyped_storage()).cpu().view(torch.int32)
+        assert a.is_contiguous()
+    assert torch.equal(got["cpu"], got["cuda"]) and torch.equal(got["cpu"], got["strided"])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("basis,level", [("def2-svp", 1), ("def2-svp", 2), ("6-31g*", 1), ("6-31g*", 2)])
 def test_rho_and_grid_energies(basis, level):
     from graddft_amd import B3LYP_GRID
