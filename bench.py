@@ -664,9 +664,9 @@ def train_batch_bench(args):
     one training step = mse_energy_loss over args.train_cycles-cycle differentiable SCF loops,
     forward + reverse to d loss / d theta, with the XC evaluation of every cycle batched over
     the molecules (batched_diff_scf_loop: one MLP pass over all grid points, ragged AO-side
-    launches).  One warm-up and one timed step per precision.  Roofline: W_pt = n_s 32 n^2 +
-    6 F_mlp flops per grid point and cycle (forward, SCF adjoint with the second-order pass;
-    n_s = 2) at the precision's peak.  Runs: FP64; the mixed precision in every cycle
+    launches).  One warm-up and one timed step per precision.  Roofline: grid_work of two density and
+    two V_xc passes of both spins and 6 F_mlp a grid point and cycle (forward, SCF adjoint with the
+    second-order pass), the last cycle at FP64 where it runs there.  Runs: FP64; the mixed precision in every cycle
     (refine_cycles=0); and the mixed precision with the loops' default last FP64 cycle.  The
     molecules start from self-consistent B3LYP densities (--batch-init b3lyp, as the
     reference's molecules carry a converged PySCF density) or the core guess.  Per molecule,
@@ -699,14 +699,19 @@ def train_batch_bench(args):
     cyc = args.train_cycles
     npts = [m.grid_size for m in mols]
     ns = [m.nao for m in mols]
-    flops = sum(N * cyc * (2 * 32 * n * n + 6 * spec.flops_per_point()) for N, n in zip(npts, ns))
+    def work(cycles, prec):
+        total = {}
+        for N, n in zip(npts, ns):
+            for u, fl in grid_work(N * cycles, n, 4, 4, 6 * spec.flops_per_point(), prec).items():
+                total[u] = total.get(u, 0) + fl
+        return total
+
     out = {"workload": f"{len(mols)} alkanes C_nH_2n+2, n_C ~ U{{1..{args.batch_max_nc}}} (seeded), def2-SVP (nao "
                        f"{min(ns)}-{max(ns)}), level-2 grids ({sum(npts)} pts in total), neural B3LYP MLP 3x128, "
                        f"mse_energy_loss over {cyc}-cycle diff_scf_loops, forward + reverse, XC batched per cycle",
            "n_molecules": len(mols), "npts_total": sum(npts), "molecule_build_s": round(t_build, 1),
            "initial_density": "self-consistent B3LYP (device CDIIS, converged_molecule)" if args.batch_init == "b3lyp" else "core Hamiltonian",
-           "initial_density_s": round(t_init, 1),
-           "flops_per_step": int(flops)}
+           "initial_density_s": round(t_init, 1)}
     grads, energies = {}, {}
     runs = [("fp64", "fp64", 0)]
     if args.precision != "fp64":
@@ -733,11 +738,11 @@ def train_batch_bench(args):
         loss, g, E = step()
         torch.cuda.synchronize()
         dt = time.perf_counter() - t1
-        peak = 78.6e12 if prec == "fp64" else 157.3e12
+        w, last = work(cyc - refine, prec), work(refine, "fp64")
+        w = {u: w.get(u, 0) + last.get(u, 0) for u in PEAK if w.get(u, 0) + last.get(u, 0)}
         grads[key] = g.cpu().numpy()
         energies[key] = E.cpu().numpy()
-        out[key] = {"s_per_step": round(dt, 3), "loss": loss, "peak_tflops": peak / 1e12,
-                    "achieved_tflops": round(flops / dt / 1e12, 2), "roofline_frac": round(flops / peak / dt, 4),
+        out[key] = {"s_per_step": round(dt, 3), "loss": loss, **against_floor(w, dt),
                     "grid_pts_cycles_per_s": round(sum(npts) * cyc / dt, 1), "refine_cycles": refine}
         if key != "fp64":
             g0 = grads["fp64"]
