@@ -18,8 +18,8 @@
 // while they are staged into LDS, as fragments of 8 consecutive k so that a lane's operand is one
 // 16-byte read.  Blocks cover all h output features, so no activation is split twice.
 //
-// 135k rows, h = 256, against 128 x 128 FP32 MFMA tiles: forward 177 -> 124 us, backward 190 -> 133,
-// weight gradient 162 -> 119 (the bytes take 53 us, 80 with the ELU outputs, the six products 47 at
+// 135k rows, h = 256, against 128 x 128 FP32 MFMA tiles: forward 177 -> 139 us (124 without the leading
+// product's own sum), backward 190 -> 135, weight gradient 162 -> 117 (the bytes take 53 us, 80 with the ELU outputs, the six products 47 at
 // the MFMA rate): two waves a SIMD do not hide all of the LDS and L2 latency between barriers.
 #pragma once
 #include "gdx_common.h"

@@ -611,9 +611,9 @@ __global__ __launch_bounds__(NT) void point_hvp_bwd_kernel(const double* __restr
 constexpr int NUM_CU = 256;    // MI355X compute units
 constexpr int RED_GROUPS = 32; // slice groups of the first reduction stage
 
-// Tiling and chunks of one molecule in slabs of `slab` points, with about `budget` work items an XCD (spins counted): every class
-// of items starts with eight chunks, one an XCD, and the class whose items cost most gets eight more
-// while they fit; chunks are not under 128 points, below which the nP x nP partials outweigh the
+// Tiling and chunks of one molecule in slabs of `slab` points, with about `budget` work items an XCD
+// (spins counted): every class of items starts with eight chunks, one an XCD, and the class whose items
+// cost most gets eight more while they fit; chunks are not under 128 points, below which the nP x nP partials outweigh the
 // products.  FP32 spreads the blocks evenly over the tiles, FP64 keeps full tiles and one ragged tile
 // (n = 96: 64 + 32, whose products divide over four waves; those of 48 + 48 do not).
 template <typename T>
@@ -655,8 +655,9 @@ inline int vxc_slots(bool fp64) { return NUM_CU / 8 * (fp64 ? 2 : 4); }
 inline size_t vxc_z_bytes(int slab, int nP, int nsv) { return (size_t)nsv * slab * nP * 4; }
 // FP32: slabs of points, so that their Z takes no more than the MLP deltas over which it lies, or than
 // ZCAP (zbytes gives the scratch for a number of slabs).  Z of the whole grid was 2.0 GB at n = 560, 427k
-// points; V_xc of both spins takes 13.3 ms there with it, 11.8 in slabs of 128 MB (they stay in the
-// last-level cache), and level within 1% at n = 82 .. 280; slabs of 64 MB cost 5 to 9% at n = 102 .. 280.
+// points.  Backward pass of a 2 x 32 network (V_xc of both spins) there 13.3 ms with all of Z, 11.8 in slabs
+// of 128 MB, which stay in the last-level cache; within 1% at n = 82 .. 280, where slabs of 64 MB cost 5 to
+// 9%.
 constexpr size_t ZCAP = (size_t)128 << 20;
 inline int vxc_slab(int Np, int nslab) { return ((Np + nslab - 1) / nslab + 63) / 64 * 64; }
 template <typename F>
