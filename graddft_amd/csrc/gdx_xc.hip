@@ -1029,7 +1029,10 @@ void launch_vxc_group(const Ctx& c, const VxcMol* mols, const VxcMol& one, const
   const size_t rows = (size_t)c.d.npts_pad;
   if constexpr (sizeof(T) == 4) {
     for (int slab = 0; slab < G.nslab; ++slab) {
-      GDX_LAUNCH("vxc_zform", vxc_zform_kernel, dim3(G.zblocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
+      if (c.d.precision & GDX_AO_LOW)
+        GDX_LAUNCH("vxc_zform", vxc_zform_kernel<true>, dim3(G.zblocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
+      else
+        GDX_LAUNCH("vxc_zform", vxc_zform_kernel<false>, dim3(G.zblocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
       GDX_LAUNCH(nm, vxc_f32_kernel, dim3(G.blocks), dim3(NT), 0, st, mols, G.nmol, one, vpt, rows, nsv, slab);
     }
   } else {

@@ -39,9 +39,10 @@ enum {
  *  GDX_BF16X6 the same kernels as GDX_FP32. */
 enum { GDX_FP64 = 0, GDX_FP32 = 1, GDX_BF16X6 = 2 };
 /* Or-ed into GDX_FP32 or GDX_BF16X6: the buffer of the five float AO planes goes on with a plane
- * (npts_pad, nao_pad) of bf16 values phi - (float)phi, with which rho is formed.  Without it the
- * rounding of phi moves E_xc by up to 2e-8 of itself: the core functions are nearly constant on every
- * shell of grid points around a nucleus, so that it does not average out. */
+ * (npts_pad, nao_pad) of bf16 values phi - (float)phi, with which rho and the v_rho phi phi^T of dE/dD
+ * are formed.  Without it the rounding of phi moves E_xc by up to 2e-8 of itself and the core's diagonal
+ * of dE/dD by 1e-7: the core functions are nearly constant on every shell of grid points around a
+ * nucleus, so that it does not average out. */
 enum { GDX_AO_LOW = 16 };
 
 /* Functional kinds evaluated on the grid.

@@ -91,3 +91,42 @@ def test_batch_energies_of_a_network(basis, level, h, layers, seed):
     # E_xc, a quarter of the energy or less, is left 3e-9 by the planes (above) and as much by the
     # roundings within the network; they have no common sign
     assert float(off.abs().max()) <= 1e-9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("restricted", [True, False])
+@pytest.mark.parametrize("n,npts", [(1, 256), (7, 512), (48, 4096), (100, 4352)])
+def test_potential_of_a_core_function(n, npts, restricted):
+    """A function that is the same on every point and lies between two FP32 numbers, as a core function
+    does on a shell: the matrix element of its square carries twice the rounding of phi, 1.1e-7, unless
+    the remainder enters with Z."""
+    from graddft_amd import B3LYP_GRID
+    from graddft_amd.molecule import Grid, Molecule
+    print(f"case: {n} functions, {npts} points, restricted={restricted}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    cols = (n + 15) // 16 * 16
+    planes = torch.zeros((5, npts, cols), dtype=torch.float64, device="cuda")
+    planes[:, :, :n] = torch.randn((5, npts, n), dtype=torch.float64, device="cuda", generator=g) / n
+    planes[:, :, n - 1] = 0.0
+    planes[0, :, n - 1] = 1.0 + 0.47 * 2.0 ** -23
+    w = torch.rand(npts, dtype=torch.float64, device="cuda", generator=g) + 0.1
+    c = torch.randn((2, n, n // 3 + 1), dtype=torch.float64, device="cuda", generator=g)
+    D = c @ c.transpose(1, 2) / n
+    D[:, n - 1, n - 1] += 1.0
+    if restricted:
+        D = D[:1].expand(2, n, n).contiguous()
+    z = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    m = Molecule(grid=Grid(torch.zeros((npts, 3), dtype=torch.float64, device="cuda"), w, w), atom_index=torch.ones(1),
+                 nuclear_pos=torch.zeros((1, 3)), ao_planes=planes, rdm1=D, nuclear_repulsion=0.0, h1e=z, s1e=z,
+                 mo_coeff=torch.zeros((2, n, n)), mo_occ=torch.zeros((2, n)), mo_energy=torch.zeros((2, n)),
+                 restricted=restricted)
+    V = {}
+    for p in ("fp64", "fp32", "bf16x6"):
+        Dg = D.detach().requires_grad_(True)
+        V[p] = torch.autograd.grad(B3LYP_GRID.xc_energy(None, m, p, rdm1=Dg), [Dg])[0][:, n - 1, n - 1]
+    for p in ("fp32", "bf16x6"):
+        off = (V[p] / V["fp64"] - 1).abs()
+        print("  ", p, off.tolist(), flush=True)
+        # Z's rounding differs from point to point; the matrix instruction's cut and the split's left
+        # out products are 2^-26 each at most
+        assert float(off.max()) <= 2.0 ** -25
